@@ -5,6 +5,7 @@
 
 #include "device/fields.hpp"
 #include "device/gemm_nt.hpp"
+#include "device/gemm_tn.hpp"
 #include "device/mlp.hpp"
 #include "device/mlp_fused.hpp"
 #include "device/surrogate.hpp"
@@ -16,6 +17,9 @@ using lm::u16;
 
 __global__ void __launch_bounds__(256) gemm_kernel(lm::GemmParams P) { lm::gemm_body(P); }
 __global__ void __launch_bounds__(256) gemm_nt_kernel(lm::GemmParams P) { lm::gemm_nt_body(P); }
+__global__ void __launch_bounds__(256) gemm_tn_kernel(lm::GemmParams P) {
+    lm::gemm_tn_body(P, lm::gemm_tn_work((int)blockIdx.x, (int)gridDim.x));
+}
 
 __global__ void __launch_bounds__(256) features_kernel(ls::SurrogateIO S) { ls::features_body(S); }
 __global__ void __launch_bounds__(256) mlp_pack_kernel(const float* W, int K, u16* dst) { lm::mlp_pack_body(W, K, dst); }
@@ -385,6 +389,8 @@ hipError_t sg_gemm(const lm::GemmParams& P, int splits, hipStream_t s) {
         dim3 grid((P.M + LM_NT_BM - 1) / LM_NT_BM, P.N / LM_NT_BN, 1);
         return hipLaunchKernel((const void*)&gemm_nt_kernel, grid, dim3(256), args, 0, s);
     }
+    if (lm::gemm_tn_applies(P))  // the weight gradients' layout: register-transposed 128 x 128 tiles
+        return hipLaunchKernel((const void*)&gemm_tn_kernel, dim3(lm::gemm_tn_tiles(P) * splits), dim3(256), args, 0, s);
     dim3 grid((P.M + LM_BM - 1) / LM_BM, (P.N + LM_BN - 1) / LM_BN, splits);
     return hipLaunchKernel((const void*)&gemm_kernel, grid, dim3(256), args, 0, s);
 }
