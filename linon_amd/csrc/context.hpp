@@ -49,8 +49,6 @@ struct Surrogate {
     float* vW[5] = {};
     float* mb[5] = {};
     float* vb[5] = {};
-    float* gW[5] = {};
-    float* gb[5] = {};
     unsigned short* Wt[4] = {};  // BF16 copies [N][K] of the hidden layers
     unsigned short* d_wpack = nullptr;  // the hidden layers in MFMA fragment order (fused inference)
     float* d_freqs = nullptr;
@@ -63,7 +61,8 @@ struct Surrogate {
     unsigned short* d_act[5] = {};
     float* d_z[4] = {};
     float *d_out = nullptr, *d_dout = nullptr, *d_err = nullptr, *d_part = nullptr, *d_loss = nullptr;
-    unsigned short* d_dz[2] = {};
+    unsigned short* d_dz[4] = {};  // the hidden layers' dZ
+    float *d_col_part = nullptr, *d_out_part = nullptr;  // row sums of the bias and output-layer gradients
     // frame
     int frame_px = 0;
     float* f_entry = nullptr;

@@ -55,7 +55,7 @@ float host_bf16_round(float x) {
 
 void Surrogate::release() {
     for (int l = 0; l < 5; ++l)
-        for (float** p : {&W[l], &b[l], &mW[l], &vW[l], &mb[l], &vb[l], &gW[l], &gb[l]}) {
+        for (float** p : {&W[l], &b[l], &mW[l], &vW[l], &mb[l], &vb[l]}) {
             if (*p) (void)hipFree(*p);
             *p = nullptr;
         }
@@ -65,7 +65,7 @@ void Surrogate::release() {
     }
     void* bufs[] = {d_wpack, d_freqs, d_states, d_targets, d_bstates, d_btargets, d_tscaled, d_bfine, d_feat, d_act[0],
                     d_act[1], d_act[2], d_act[3], d_act[4], d_z[0], d_z[1], d_z[2], d_z[3], d_out, d_dout, d_err,
-                    d_dz[0], d_dz[1], d_part, d_loss, f_entry, f_entered, f_states, f_texel, f_count, f_pred,
+                    d_dz[0], d_dz[1], d_dz[2], d_dz[3], d_col_part, d_out_part, d_part, d_loss, f_entry, f_entered, f_states, f_texel, f_count, f_pred,
                     f_accepted, f_list, f_exits, f_errs, f_feat, f_act0, f_act1, f_out, f_steps, f_base, f_mask};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
@@ -85,8 +85,6 @@ linon_status Context::surrogate_alloc_params() {
         LS_CHECK(this, dalloc(S.vW[l], (size_t)K * N));
         LS_CHECK(this, dalloc(S.mb[l], N));
         LS_CHECK(this, dalloc(S.vb[l], N));
-        LS_CHECK(this, dalloc(S.gW[l], (size_t)K * N));
-        LS_CHECK(this, dalloc(S.gb[l], N));
         LS_CHECK(this, hipMemset(S.mW[l], 0, (size_t)K * N * 4));
         LS_CHECK(this, hipMemset(S.vW[l], 0, (size_t)K * N * 4));
         LS_CHECK(this, hipMemset(S.mb[l], 0, N * 4));
@@ -311,14 +309,15 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
     LS_CHECK(this, dalloc(S.d_out, (size_t)B * LS_OUT));
     LS_CHECK(this, dalloc(S.d_dout, (size_t)B * LS_OUT));
     LS_CHECK(this, dalloc(S.d_err, (size_t)B));
-    LS_CHECK(this, dalloc(S.d_dz[0], (size_t)B * LS_HIDDEN));
-    LS_CHECK(this, dalloc(S.d_dz[1], (size_t)B * LS_HIDDEN));
+    for (int l = 0; l < 4; ++l) LS_CHECK(this, dalloc(S.d_dz[l], (size_t)B * LS_HIDDEN));
     const int ksplit = 1024;  // batch rows per split-K chunk of a weight gradient
     const int splits = (B + ksplit - 1) / ksplit;
-    // one [K][LS_HIDDEN] partial per split, for the widest K of the four layers
-    const int max_k = *std::max_element(kLayerK, kLayerK + 4);
-    const size_t part_elems = (size_t)splits * max_k * LS_HIDDEN;
-    LS_CHECK(this, dalloc(S.d_part, part_elems));
+    // one [K][LS_HIDDEN] partial per split and layer
+    size_t part_at[5] = {0};
+    for (int l = 0; l < 4; ++l) part_at[l + 1] = part_at[l] + (size_t)splits * kLayerK[l] * LS_HIDDEN;
+    LS_CHECK(this, dalloc(S.d_part, part_at[4]));
+    LS_CHECK(this, dalloc(S.d_col_part, (size_t)4 * LM_SUM_ROWS * LS_HIDDEN));
+    LS_CHECK(this, dalloc(S.d_out_part, (size_t)LM_SUM_ROWS * (LS_HIDDEN + 1) * LS_OUT));
     LS_CHECK(this, dalloc(S.d_loss, 1));
 
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -338,66 +337,74 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
         if (want_loss) LS_CHECK(this, hipMemsetAsync(S.d_loss, 0, 4, s));
         LS_CHECK(this, sg_loss(S.d_out, S.d_btargets, S.d_bfine, B, S.scale_p, cfg.tolerance, conf_w, S.d_dout,
                                S.d_err, S.d_loss, s));
-        // output layer (FP32)
-        LS_CHECK(this, sg_out_layer_grad(S.d_act[4], S.d_dout, B, S.gW[4], S.gb[4], s));
-        LS_CHECK(this, sg_out_layer_back(S.d_dout, S.W[4], S.d_z[3], B, S.d_dz[0], s));
-        // hidden layers, top down; dz[cur] holds dZ of layer l
-        int cur = 0;
-        for (int l = 3; l >= 0; --l) {
+        // output layer (FP32), then the hidden layers, top down: each layer's dZ
+        LS_CHECK(this, sg_out_layer_back(S.d_dout, S.W[4], S.d_z[3], B, S.d_dz[3], s));
+        for (int l = 3; l > 0; --l) {  // dZ of layer l-1 = (dZ W^T) * silu'(z_{l-1})
             const int K = kLayerK[l];
-            if ((size_t)splits * K * LS_HIDDEN > part_elems)
-                return fail(LINON_ERR_STATE, "surrogate: split-K partial buffer too small");
-            lm::GemmParams G;  // dW = X^T dZ, split over the batch
-            std::memset(&G, 0, sizeof(G));
-            G.A = acts[l];
-            G.B = S.d_dz[cur];
-            G.M = K;
-            G.N = LS_HIDDEN;
-            G.K = B;
-            G.lda = K;
-            G.ldb = LS_HIDDEN;
-            G.a_trans = 1;
-            G.b_trans = 0;
-            G.k_per_split = ksplit;
-            G.epi = LM_EPI_PARTIAL;
-            G.out_f32 = S.d_part;
-            G.ldc = LS_HIDDEN;
-            LS_CHECK(this, sg_gemm(G, splits, s));
-            LS_CHECK(this, sg_reduce(S.d_part, splits, K * LS_HIDDEN, S.gW[l], s));
-            LS_CHECK(this, sg_colsum(S.d_dz[cur], B, LS_HIDDEN, S.gb[l], s));
-            if (l > 0) {  // dZ of layer l-1 = (dZ W^T) * silu'(z_{l-1})
-                lm::GemmParams D;
-                std::memset(&D, 0, sizeof(D));
-                D.A = S.d_dz[cur];
-                D.B = S.Wt[l];
-                D.M = B;
-                D.N = K;
-                D.K = LS_HIDDEN;
-                D.lda = LS_HIDDEN;
-                D.ldb = K;
-                D.a_trans = 0;
-                D.b_trans = 0;
-                D.k_per_split = LS_HIDDEN;
-                D.epi = LM_EPI_SILU_GRAD;
-                D.z_in = S.d_z[l - 1];
-                D.out_bf16 = S.d_dz[cur ^ 1];
-                D.ldc = K;
-                LS_CHECK(this, sg_gemm(D, 1, s));
-                cur ^= 1;
-            }
+            lm::GemmParams D;
+            std::memset(&D, 0, sizeof(D));
+            D.A = S.d_dz[l];
+            D.B = S.Wt[l];
+            D.M = B;
+            D.N = K;
+            D.K = LS_HIDDEN;
+            D.lda = LS_HIDDEN;
+            D.ldb = K;
+            D.a_trans = 0;
+            D.b_trans = 0;
+            D.k_per_split = LS_HIDDEN;
+            D.epi = LM_EPI_SILU_GRAD;
+            D.z_in = S.d_z[l - 1];
+            D.out_bf16 = S.d_dz[l - 1];
+            D.ldc = K;
+            LS_CHECK(this, sg_gemm(D, 1, s));
         }
-        // Adam, the learning rate on a cosine from lr down to lr / 100 over the run
+        // every gradient, then Adam
+        lm::GradParams G;
+        std::memset(&G, 0, sizeof(G));
+        for (int l = 0; l < 4; ++l) {  // dW = X^T dZ, split over the batch
+            lm::GemmParams& D = G.dw[l];
+            D.A = acts[l];
+            D.B = S.d_dz[l];
+            D.M = kLayerK[l];
+            D.N = LS_HIDDEN;
+            D.K = B;
+            D.lda = kLayerK[l];
+            D.ldb = LS_HIDDEN;
+            D.a_trans = 1;
+            D.b_trans = 0;
+            D.k_per_split = ksplit;
+            D.epi = LM_EPI_PARTIAL;
+            D.out_f32 = S.d_part + part_at[l];
+            D.ldc = LS_HIDDEN;
+        }
+        G.splits = splits;
+        G.rows = B;
+        G.act_top = S.d_act[4];
+        G.dout = S.d_dout;
+        G.col_part = S.d_col_part;
+        G.out_part = S.d_out_part;
+        LS_CHECK(this, sg_grads(G, s));
+        // the learning rate on a cosine from lr down to lr / 100 over the run
         ++S.adam_t;
         const float bc1 = 1.0f - std::pow(b1, (float)S.adam_t), bc2 = 1.0f - std::pow(b2, (float)S.adam_t);
         const float lr = cfg.lr * (0.01f + 0.99f * 0.5f * (1.0f + std::cos(3.14159265f * step / std::max(1, cfg.steps))));
-        for (int l = 0; l < 5; ++l) {
-            const int K = l < 4 ? kLayerK[l] : LS_HIDDEN;
-            const int Nn = l < 4 ? LS_HIDDEN : LS_OUT;
-            LS_CHECK(this, sg_adam(S.W[l], S.mW[l], S.vW[l], S.gW[l], K, Nn, lr, b1, b2, eps, bc1, bc2,
-                                   l < 4 ? S.Wt[l] : nullptr, K, s));
-            LS_CHECK(this, sg_adam(S.b[l], S.mb[l], S.vb[l], S.gb[l], 1, Nn, lr, b1, b2, eps, bc1, bc2, nullptr, 0,
-                                   s));
-        }
+        lm::UpdateParams U;
+        std::memset(&U, 0, sizeof(U));
+        for (int l = 0; l < 4; ++l)
+            U.hidden[l] = lm::LayerUpdate{S.W[l], S.mW[l], S.vW[l], S.b[l], S.mb[l], S.vb[l], S.Wt[l],
+                                          S.d_part + part_at[l], kLayerK[l]};
+        U.w = S.W[4];
+        U.m = S.mW[4];
+        U.v = S.vW[4];
+        U.b = S.b[4];
+        U.mb = S.mb[4];
+        U.vb = S.vb[4];
+        U.col_part = S.d_col_part;
+        U.out_part = S.d_out_part;
+        U.splits = splits;
+        U.adam = lm::AdamStep{lr, b1, b2, eps, bc1, bc2};
+        LS_CHECK(this, sg_update(U, s));
         if (want_loss) {
             LS_CHECK(this, hipMemcpyAsync(&last_loss, S.d_loss, 4, hipMemcpyDeviceToHost, s));
             LS_CHECK(this, hipStreamSynchronize(s));

@@ -9,6 +9,7 @@
 #include "device/mlp.hpp"
 #include "device/mlp_fused.hpp"
 #include "device/surrogate.hpp"
+#include "device/train.hpp"
 #include "surrogate_kernels.hpp"
 
 namespace LINON_KERNEL_NS {
@@ -20,6 +21,8 @@ __global__ void __launch_bounds__(256) gemm_nt_kernel(lm::GemmParams P) { lm::ge
 __global__ void __launch_bounds__(256) gemm_tn_kernel(lm::GemmParams P) {
     lm::gemm_tn_body(P, lm::gemm_tn_work((int)blockIdx.x, (int)gridDim.x));
 }
+__global__ void __launch_bounds__(256) grads_kernel(lm::GradParams P) { lm::grads_body(P); }
+__global__ void __launch_bounds__(LM_SUM_ROWS) update_kernel(lm::UpdateParams P) { lm::update_body(P); }
 
 __global__ void __launch_bounds__(256) features_kernel(ls::SurrogateIO S) { ls::features_body(S); }
 __global__ void __launch_bounds__(256) mlp_pack_kernel(const float* W, int K, u16* dst) { lm::mlp_pack_body(W, K, dst); }
@@ -209,33 +212,6 @@ __global__ void __launch_bounds__(256) out_layer_back_kernel(const float* dout, 
     dz[t] = lm::f2bf(s * lm::silu_grad(z[t]));
 }
 
-// Output-layer weight/bias gradients: one block per k (0..LS_HIDDEN, where k == LS_HIDDEN is
-// the bias), reducing over the batch.
-__global__ void __launch_bounds__(256) out_layer_grad_kernel(const u16* act, const float* dout, int n, float* dW,
-                                                             float* db) {
-    const int k = blockIdx.x;
-    float s[LS_OUT];
-    for (int o = 0; o < LS_OUT; ++o) s[o] = 0.0f;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const float a = (k < LS_HIDDEN) ? lm::bf2f(act[(size_t)i * LS_HIDDEN + k]) : 1.0f;
-        for (int o = 0; o < LS_OUT; ++o) s[o] = __builtin_fmaf(a, dout[(size_t)i * LS_OUT + o], s[o]);
-    }
-    __shared__ float red[LS_OUT][256];
-    for (int o = 0; o < LS_OUT; ++o) red[o][threadIdx.x] = s[o];
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-            for (int o = 0; o < LS_OUT; ++o) red[o][threadIdx.x] += red[o][threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x < LS_OUT) {
-        if (k < LS_HIDDEN)
-            dW[k * LS_OUT + threadIdx.x] = red[threadIdx.x][0];
-        else
-            db[threadIdx.x] = red[threadIdx.x][0];
-    }
-}
-
 // Sums split-K partials: out[j] = sum_s part[s][j].
 __global__ void __launch_bounds__(256) reduce_partials_kernel(const float* part, int splits, int n, float* out) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -243,40 +219,6 @@ __global__ void __launch_bounds__(256) reduce_partials_kernel(const float* part,
     float s = 0.0f;
     for (int k = 0; k < splits; ++k) s += part[(size_t)k * n + j];
     out[j] = s;
-}
-
-// Bias gradient of a hidden layer: column sums of bf16 dZ [n][cols].
-__global__ void __launch_bounds__(256) colsum_kernel(const u16* dz, int n, int cols, float* out) {
-    const int c = blockIdx.x;
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += lm::bf2f(dz[(size_t)i * cols + c]);
-    __shared__ float red[256];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = red[0];
-}
-
-// Adam on FP32 master weights [K][N]; optionally refreshes the bf16 transposed copy [N][ldt].
-__global__ void __launch_bounds__(256) adam_kernel(float* w, float* m, float* v, const float* g, int K, int N,
-                                                   float lr, float b1, float b2, float eps, float bc1, float bc2,
-                                                   u16* wt, int ldt) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= K * N) return;
-    const float gr = g[t];
-    const float mm = b1 * m[t] + (1.0f - b1) * gr;
-    const float vv = b2 * v[t] + (1.0f - b2) * gr * gr;
-    m[t] = mm;
-    v[t] = vv;
-    const float nw = w[t] - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
-    w[t] = nw;
-    if (wt) {
-        const int k = t / N, n = t % N;
-        wt[(size_t)n * ldt + k] = lm::f2bf(nw);
-    }
 }
 
 // Surrogate verdict per entered ray: accept (write the exit point to the mapping) when the
@@ -439,21 +381,16 @@ hipError_t sg_out_layer_back(const float* dout, const float* W, const float* z, 
     hipLaunchKernelGGL(out_layer_back_kernel, LS_GRID(n * LS_HIDDEN), 0, s, dout, W, z, n, dz);
     return hipGetLastError();
 }
-hipError_t sg_out_layer_grad(const u16* act, const float* dout, int n, float* dW, float* db, hipStream_t s) {
-    hipLaunchKernelGGL(out_layer_grad_kernel, dim3(LS_HIDDEN + 1), dim3(256), 0, s, act, dout, n, dW, db);
-    return hipGetLastError();
-}
 hipError_t sg_reduce(const float* part, int splits, int n, float* out, hipStream_t s) {
     hipLaunchKernelGGL(reduce_partials_kernel, LS_GRID(n), 0, s, part, splits, n, out);
     return hipGetLastError();
 }
-hipError_t sg_colsum(const u16* dz, int n, int cols, float* out, hipStream_t s) {
-    hipLaunchKernelGGL(colsum_kernel, dim3(cols), dim3(256), 0, s, dz, n, cols, out);
+hipError_t sg_grads(const lm::GradParams& P, hipStream_t s) {
+    hipLaunchKernelGGL(grads_kernel, dim3(lm::grads_sum_blocks() + lm::grads_tiles(P)), dim3(256), 0, s, P);
     return hipGetLastError();
 }
-hipError_t sg_adam(float* w, float* m, float* v, const float* g, int K, int N, float lr, float b1, float b2, float eps,
-                   float bc1, float bc2, u16* wt, int ldt, hipStream_t s) {
-    hipLaunchKernelGGL(adam_kernel, LS_GRID(K * N), 0, s, w, m, v, g, K, N, lr, b1, b2, eps, bc1, bc2, wt, ldt);
+hipError_t sg_update(const lm::UpdateParams& P, hipStream_t s) {
+    hipLaunchKernelGGL(update_kernel, dim3(lm::update_blocks(P)), dim3(LM_SUM_ROWS), 0, s, P);
     return hipGetLastError();
 }
 hipError_t sg_accept(const float* out, const float* base, const int* texel_of, int n, const int* n_dev, float scale_p,

@@ -5,6 +5,7 @@
 #include "device/mlp.hpp"
 #include "device/mlp_fused.hpp"
 #include "device/surrogate.hpp"
+#include "device/train.hpp"
 
 // Compiled twice like kernels.hip: LINON_KERNEL_NS is linon (IEEE) or linon_wgslmath (WGSL
 // accuracy); the RK4 legs of a surrogate frame use the build the plain kernel of that field uses.
@@ -28,11 +29,9 @@
     hipError_t sg_loss(const float* out, const float* target, const float* fine, int n, float scale_p, float tol, \
                        float conf_weight, float* dout, float* err, float* loss_sum, hipStream_t s); \
     hipError_t sg_out_layer_back(const float* dout, const float* W, const float* z, int n, lm::u16* dz, hipStream_t s); \
-    hipError_t sg_out_layer_grad(const lm::u16* act, const float* dout, int n, float* dW, float* db, hipStream_t s); \
     hipError_t sg_reduce(const float* part, int splits, int n, float* out, hipStream_t s); \
-    hipError_t sg_colsum(const lm::u16* dz, int n, int cols, float* out, hipStream_t s); \
-    hipError_t sg_adam(float* w, float* m, float* v, const float* g, int K, int N, float lr, float b1, float b2, float eps, \
-                       float bc1, float bc2, lm::u16* wt, int ldt, hipStream_t s); \
+    hipError_t sg_grads(const lm::GradParams& P, hipStream_t s); \
+    hipError_t sg_update(const lm::UpdateParams& P, hipStream_t s); \
     hipError_t sg_accept(const float* out, const float* base, const int* texel_of, int n, const int* n_dev, \
                          float scale_p, float thr, float* mapping, float* pred_exit, int* fallback, int* n_fallback, \
                          int* accepted, hipStream_t s); \
