@@ -53,15 +53,15 @@ struct Surrogate {
     unsigned short* d_wpack = nullptr;  // the hidden layers in MFMA fragment order (fused inference)
     float* d_freqs = nullptr;
     // training
-    float *d_states = nullptr, *d_targets = nullptr, *d_bstates = nullptr, *d_btargets = nullptr;
+    float *d_states = nullptr, *d_targets = nullptr;
     float* d_tscaled = nullptr;  // network targets (exit - coarse exit) * scale
-    float* d_bfine = nullptr;    // the mini-batch's RK4 exits
     float scale_p = 0.5f, scale_d = 1.0f;  // output scales of the exit point and direction
+    unsigned short* d_bpack = nullptr;     // layers 1..3 transposed, in fragment order (backward pass)
     unsigned short* d_feat = nullptr;
-    unsigned short* d_act[5] = {};
-    float* d_z[4] = {};
-    float *d_out = nullptr, *d_dout = nullptr, *d_err = nullptr, *d_part = nullptr, *d_loss = nullptr;
-    unsigned short* d_dz[4] = {};  // the hidden layers' dZ
+    unsigned short* d_act[4] = {};         // the hidden layers' outputs
+    unsigned short* d_dz[4] = {};          // and their dZ
+    float* d_z = nullptr;                  // pre-activations of layers 0..2, in register order
+    float *d_dout = nullptr, *d_part = nullptr, *d_loss = nullptr;
     float *d_col_part = nullptr, *d_out_part = nullptr;  // row sums of the bias and output-layer gradients
     // frame
     int frame_px = 0;
@@ -172,15 +172,14 @@ struct Context {
     Surrogate sg;
     linon_status surrogate_alloc_params();
     linon_status surrogate_init_params(unsigned long long seed);
-    linon_status surrogate_forward(int n, const unsigned short* feat, unsigned short* const act[5],
-                                   float* const z[4], hipStream_t s);
+    linon_status surrogate_forward(int n, const unsigned short* feat, unsigned short* const act[5], hipStream_t s);
     linon_status surrogate_train(const linon_surrogate_config& cfg, linon_surrogate_stats* stats);
     linon_status surrogate_eval(const float* states, const float* targets, const float* fine, int n,
                                 std::vector<float>& err);
     linon_status surrogate_frame(hipStream_t s);
     linon_status surrogate_collect_stats();
     linon_status surrogate_save(void* out, size_t capacity, size_t* needed);
-    linon_status surrogate_pack();  // refreshes d_wpack from the master weights
+    linon_status surrogate_pack();  // fills d_wpack from the master weights
     linon_status surrogate_infer(const float* states, int n, float* out, bool fused);
     linon_status surrogate_load(const void* data, size_t bytes);
     StepParams surrogate_step_params() const;

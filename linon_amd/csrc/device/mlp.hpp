@@ -4,9 +4,7 @@
 //     staged through LDS.  LDS holds A as [m][k] and B as [n][k] (k contiguous), so each lane
 //     reads its 8 consecutive k-values of one row / column with a single 16-byte load; the
 //     global->LDS copy absorbs either storage order of A and B (row-major or transposed).
-//   * fused epilogues: bias + SiLU (+ the pre-activation kept for the backward pass), plain
-//     bias (output layer), SiLU' gating of the backward pass, and split-K partial sums for
-//     weight gradients.
+//   * fused epilogues: bias + SiLU (+ the pre-activation), plain bias, and split-K partial sums.
 // Operand layout of v_mfma_f32_32x32x16_bf16 for lane l: A row (l % 32), k 8*(l/32)..+7; B
 // column (l % 32), same k; D[i][j] in VGPR r: j = l % 32, i = 8*(r/4) + 4*(l/32) + r%4.
 #pragma once
@@ -27,8 +25,7 @@ typedef unsigned short u16;
 // epilogue kinds
 #define LM_EPI_STORE_F32 0      // C (+bias) -> fp32 out
 #define LM_EPI_BIAS_SILU 1      // Z = C + bias -> z_out (fp32), A = silu(Z) -> bf16 out
-#define LM_EPI_SILU_GRAD 2      // dZ = C * silu'(Z_in) -> bf16 out (and fp32 copy when out_f32)
-#define LM_EPI_PARTIAL 3        // split-K partial: fp32 out + blockIdx.z * M * N
+#define LM_EPI_PARTIAL 2        // split-K partial: fp32 out + blockIdx.z * M * N
 
 struct GemmParams {
     const u16* A;   // bf16 bits
@@ -40,7 +37,6 @@ struct GemmParams {
     int k_per_split;  // split-K chunk (multiple of LM_BK); = K when no split
     int epi;
     const float* bias;   // [N]
-    const float* z_in;   // [M][N] fp32 pre-activations (LM_EPI_SILU_GRAD)
     float* out_f32;      // [M][N] (or partials)
     u16* out_bf16;       // [M][N]
     float* z_out;        // [M][N] fp32 pre-activations (LM_EPI_BIAS_SILU)
@@ -146,12 +142,6 @@ __device__ __forceinline__ void gemm_body(const GemmParams& P) {
                 float z = c + P.bias[j];
                 if (P.z_out) P.z_out[o] = z;
                 P.out_bf16[o] = f2bf(silu(z));
-                break;
-            }
-            case LM_EPI_SILU_GRAD: {
-                float g = c * silu_grad(P.z_in[o]);
-                P.out_bf16[o] = f2bf(g);
-                if (P.out_f32) P.out_f32[o] = g;
                 break;
             }
             default:  // LM_EPI_PARTIAL

@@ -37,16 +37,24 @@ __host__ __device__ inline size_t pack_offset(int layer) {
     return layer == 0 ? 0 : (size_t)LM_PACK_LAYER0 + (size_t)(layer - 1) * LM_PACK_LAYER;
 }
 
-// Packs one hidden layer's FP32 master weights W [K][256] into MFMA B fragments: element e of
-// fragment (ks, ct, lane) is bf16(W[16 ks + 8 (lane / 32) + e][32 ct + lane % 32]), i.e. what
-// lane `lane` supplies as B (k 8 (lane / 32) .. +7 of column lane % 32) for the k step ks of
-// column tile ct.  One thread per fragment.
+// A hidden layer's weights in MFMA fragment order: element e of fragment (ks, ct, lane) is what
+// lane `lane` supplies for the k step ks of column tile ct, the value of contraction index
+// 16 ks + 8 (lane / 32) + e and column 32 ct + lane % 32.  Where (k, n) stands:
+__host__ __device__ inline int pack_index(int k, int n) {
+    return (((k >> 4) * 8 + (n >> 5)) * 64 + (n & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
+}
+
+// Packs one hidden layer's FP32 master weights W [K][256] as BF16 fragments, one thread per
+// fragment: of the forward product (contraction over k), or, with Transposed, of the backward
+// product W^T (contraction over the 256 columns; K = 256).
+template <bool Transposed>
 __device__ __forceinline__ void mlp_pack_body(const float* W, int K, u16* dst) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (K / 16) * 8 * 64) return;
     const int lane = t & 63, ct = (t >> 6) & 7, ks = t >> 9;
     const int k0 = 16 * ks + 8 * (lane >> 5), n = 32 * ct + (lane & 31);
-    for (int e = 0; e < 8; ++e) dst[(size_t)t * 8 + e] = f2bf(W[(size_t)(k0 + e) * LS_HIDDEN + n]);
+    for (int e = 0; e < 8; ++e)
+        dst[(size_t)t * 8 + e] = f2bf(Transposed ? W[(size_t)n * LS_HIDDEN + k0 + e] : W[(size_t)(k0 + e) * LS_HIDDEN + n]);
 }
 
 struct MlpInferParams {

@@ -20,8 +20,7 @@
 // splits (the partials' 65 MB), where four reductions and ten Adam launches took 113.
 #pragma once
 #include "gemm_tn.hpp"
-#include "mlp.hpp"
-#include "surrogate.hpp"
+#include "mlp_fused.hpp"
 
 namespace lm {
 
@@ -159,7 +158,8 @@ __device__ __forceinline__ float adam_update(const AdamStep& A, float g, float* 
 struct LayerUpdate {
     float *w, *m, *v;     // [K][256]
     float *b, *mb, *vb;   // [256]
-    u16* wt;              // [256][K] the BF16 copy
+    u16* wpack;           // the BF16 fragments of the forward product (mlp_pack_body's order)
+    u16* bpack;           // and of the backward product, W^T; null for the first layer
     const float* part;    // [splits][K][256]
     int K;
 };
@@ -211,7 +211,9 @@ __device__ __forceinline__ void update_body(const UpdateParams& P) {
             }
             for (; s < P.splits; ++s) g += p[(size_t)s * stride];
             const float nw = adam_update(P.adam, g, L.w + j, L.m + j, L.v + j);
-            L.wt[(size_t)t * L.K + b] = f2bf(nw);
+            const u16 nb = f2bf(nw);
+            L.wpack[pack_index(b, t)] = nb;
+            if (L.bpack) L.bpack[pack_index(t, b)] = nb;
             return;
         }
         b -= L.K;

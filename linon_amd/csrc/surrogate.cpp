@@ -1,11 +1,11 @@
 // Learned flow-map surrogate: host side (training loop, frame pipeline, statistics).
 //
 // Training follows the usual data-parallel recipe on one device: uniform entry states ->
-// labels from the FP32 RK4 flow-map kernel -> mini-batches gathered by a counter-based hash ->
-// forward (four BF16-MFMA GEMMs with fused bias+SiLU, FP32 output layer) -> loss (MSE of the
-// scaled exit state + logistic loss of the confidence head against "error < tolerance") ->
-// backward (FP32 output layer, BF16-MFMA GEMMs for dX with the SiLU' gate fused, split-K GEMMs
-// for dW) -> Adam on FP32 master weights, which also refreshes the BF16 [N][K] weight copies.
+// labels from the FP32 RK4 flow-map kernel -> three launches a step: the pass (mini-batch gathered
+// by a counter-based hash, BF16-MFMA forward with bias+SiLU, FP32 output layer, loss = MSE of the
+// scaled exit state + logistic loss of the confidence head against "error < tolerance", and dZ
+// back through every layer), all gradients (split-K MFMA tiles, row sums), and their final sums
+// with Adam on the FP32 master weights, which also rewrites the BF16 weight fragments.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -63,10 +63,10 @@ void Surrogate::release() {
         if (Wt[l]) (void)hipFree(Wt[l]);
         Wt[l] = nullptr;
     }
-    void* bufs[] = {d_wpack, d_freqs, d_states, d_targets, d_bstates, d_btargets, d_tscaled, d_bfine, d_feat, d_act[0],
-                    d_act[1], d_act[2], d_act[3], d_act[4], d_z[0], d_z[1], d_z[2], d_z[3], d_out, d_dout, d_err,
-                    d_dz[0], d_dz[1], d_dz[2], d_dz[3], d_col_part, d_out_part, d_part, d_loss, f_entry, f_entered, f_states, f_texel, f_count, f_pred,
-                    f_accepted, f_list, f_exits, f_errs, f_feat, f_act0, f_act1, f_out, f_steps, f_base, f_mask};
+    void* bufs[] = {d_wpack, d_bpack, d_freqs, d_states, d_targets, d_tscaled, d_feat, d_act[0], d_act[1], d_act[2],
+                    d_act[3], d_dz[0], d_dz[1], d_dz[2], d_dz[3], d_z, d_dout, d_part, d_loss, d_col_part, d_out_part,
+                    f_entry, f_entered, f_states, f_texel, f_count, f_pred, f_accepted, f_list, f_exits, f_errs, f_feat,
+                    f_act0, f_act1, f_out, f_steps, f_base, f_mask};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : ev)
@@ -137,10 +137,9 @@ linon_status Context::surrogate_init_params(unsigned long long seed) {
     return LINON_OK;
 }
 
-// Forward of the hidden layers for n rows of features: act[0] = features, act[l+1] = silu(z).
-// With z != null the pre-activations are kept (training).
-linon_status Context::surrogate_forward(int n, const lm::u16* feat, lm::u16* const act[5], float* const z[4],
-                                        hipStream_t s) {
+// Forward of the hidden layers for n rows of features, one GEMM a layer: act[0] = features,
+// act[l+1] = silu(z).
+linon_status Context::surrogate_forward(int n, const lm::u16* feat, lm::u16* const act[5], hipStream_t s) {
     Surrogate& S = sg;
     const lm::u16* x = feat;
     for (int l = 0; l < 4; ++l) {
@@ -159,7 +158,6 @@ linon_status Context::surrogate_forward(int n, const lm::u16* feat, lm::u16* con
         P.epi = LM_EPI_BIAS_SILU;
         P.bias = S.b[l];
         P.out_bf16 = act[l + 1];
-        P.z_out = z ? z[l] : nullptr;
         P.ldc = LS_HIDDEN;
         LS_CHECK(this, sg_gemm(P, 1, s));
         x = act[l + 1];
@@ -170,13 +168,13 @@ linon_status Context::surrogate_forward(int n, const lm::u16* feat, lm::u16* con
 linon_status Context::surrogate_pack() {
     Surrogate& S = sg;
     if (!S.d_wpack) LS_CHECK(this, hipMalloc(&S.d_wpack, (size_t)LM_PACK_TOTAL * sizeof(lm::u16)));
-    for (int l = 0; l < 4; ++l) LS_CHECK(this, sg_mlp_pack(S.W[l], kLayerK[l], S.d_wpack + lm::pack_offset(l), stream));
+    for (int l = 0; l < 4; ++l) LS_CHECK(this, sg_mlp_pack(S.W[l], kLayerK[l], S.d_wpack + lm::pack_offset(l), false, stream));
     LS_CHECK(this, hipStreamSynchronize(stream));
     return LINON_OK;
 }
 
-// Raw network outputs for n states, through the fused inference kernel or the training path's
-// kernels (features, four GEMMs, output layer); both give the same bits.
+// Raw network outputs for n states, through the fused inference kernel or one kernel a layer
+// (features, four GEMMs, output layer); both give the same bits.
 linon_status Context::surrogate_infer(const float* states, int n, float* out, bool fused) {
     Surrogate& S = sg;
     if (!S.trained) return fail(LINON_ERR_STATE, "surrogate_infer: no trained surrogate");
@@ -218,7 +216,7 @@ linon_status Context::surrogate_infer(const float* states, int n, float* out, bo
             ls::SurrogateIO io{d_in, n, S.cfg.radius, S.d_freqs, feat};
             if (sg_features(io, s) != hipSuccess) { st = fail(LINON_ERR_HIP, "surrogate_infer: features"); break; }
             lm::u16* const acts[5] = {feat, a0, a1, a0, a1};
-            st = surrogate_forward(n, feat, acts, nullptr, s);
+            st = surrogate_forward(n, feat, acts, s);
             if (st != LINON_OK) break;
             if (sg_out_layer(a1, S.W[4], S.b[4], n, d_out, s) != hipSuccess) {
                 st = fail(LINON_ERR_HIP, "surrogate_infer: output layer");
@@ -300,16 +298,19 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
     auto t1 = std::chrono::steady_clock::now();
 
     // ---- buffers ----
-    LS_CHECK(this, dalloc(S.d_bstates, (size_t)B * 6));
-    LS_CHECK(this, dalloc(S.d_btargets, (size_t)B * 6));
-    LS_CHECK(this, dalloc(S.d_bfine, (size_t)B * 6));
+    const size_t tiles = ((size_t)B + LM_FUSED_ROWS - 1) / LM_FUSED_ROWS;
     LS_CHECK(this, dalloc(S.d_feat, (size_t)B * LS_FEATS_PAD));
-    for (int l = 1; l < 5; ++l) LS_CHECK(this, dalloc(S.d_act[l], (size_t)B * LS_HIDDEN));
-    for (int l = 0; l < 4; ++l) LS_CHECK(this, dalloc(S.d_z[l], (size_t)B * LS_HIDDEN));
-    LS_CHECK(this, dalloc(S.d_out, (size_t)B * LS_OUT));
+    for (int l = 0; l < 4; ++l) {
+        LS_CHECK(this, dalloc(S.d_act[l], (size_t)B * LS_HIDDEN));
+        LS_CHECK(this, dalloc(S.d_dz[l], (size_t)B * LS_HIDDEN));
+    }
+    LS_CHECK(this, dalloc(S.d_z, 3 * tiles * LM_FUSED_ROWS * LS_HIDDEN));
     LS_CHECK(this, dalloc(S.d_dout, (size_t)B * LS_OUT));
-    LS_CHECK(this, dalloc(S.d_err, (size_t)B));
-    for (int l = 0; l < 4; ++l) LS_CHECK(this, dalloc(S.d_dz[l], (size_t)B * LS_HIDDEN));
+    LS_CHECK(this, dalloc(S.d_bpack, (size_t)3 * LM_PACK_LAYER));
+    st = surrogate_pack();  // the forward fragments; each update rewrites both kinds
+    if (st != LINON_OK) return st;
+    for (int l = 1; l < 4; ++l)
+        LS_CHECK(this, sg_mlp_pack(S.W[l], LS_HIDDEN, S.d_bpack + (size_t)(l - 1) * LM_PACK_LAYER, true, s));
     const int ksplit = 1024;  // batch rows per split-K chunk of a weight gradient
     const int splits = (B + ksplit - 1) / ksplit;
     // one [K][LS_HIDDEN] partial per split and layer
@@ -324,47 +325,43 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
     const float conf_w = 0.1f;
     float last_loss = 0.0f;
     for (int step = 0; step < cfg.steps; ++step) {
-        LS_CHECK(this, sg_gather(S.d_states, S.d_tscaled, S.d_targets, n_train, cfg.seed ^ 0x5DEECE66Dull, step, B,
-                                 S.d_bstates, S.d_btargets, S.d_bfine, s));
-        ls::SurrogateIO io{S.d_bstates, B, cfg.radius, S.d_freqs, S.d_feat};
-        LS_CHECK(this, sg_features(io, s));
-        lm::u16* const acts[5] = {S.d_feat, S.d_act[1], S.d_act[2], S.d_act[3], S.d_act[4]};
-        float* const zs[4] = {S.d_z[0], S.d_z[1], S.d_z[2], S.d_z[3]};
-        st = surrogate_forward(B, S.d_feat, acts, zs, s);
-        if (st != LINON_OK) return st;
-        LS_CHECK(this, sg_out_layer(S.d_act[4], S.W[4], S.b[4], B, S.d_out, s));
         const bool want_loss = (step % 50 == 0) || step == cfg.steps - 1;
         if (want_loss) LS_CHECK(this, hipMemsetAsync(S.d_loss, 0, 4, s));
-        LS_CHECK(this, sg_loss(S.d_out, S.d_btargets, S.d_bfine, B, S.scale_p, cfg.tolerance, conf_w, S.d_dout,
-                               S.d_err, S.d_loss, s));
-        // output layer (FP32), then the hidden layers, top down: each layer's dZ
-        LS_CHECK(this, sg_out_layer_back(S.d_dout, S.W[4], S.d_z[3], B, S.d_dz[3], s));
-        for (int l = 3; l > 0; --l) {  // dZ of layer l-1 = (dZ W^T) * silu'(z_{l-1})
-            const int K = kLayerK[l];
-            lm::GemmParams D;
-            std::memset(&D, 0, sizeof(D));
-            D.A = S.d_dz[l];
-            D.B = S.Wt[l];
-            D.M = B;
-            D.N = K;
-            D.K = LS_HIDDEN;
-            D.lda = LS_HIDDEN;
-            D.ldb = K;
-            D.a_trans = 0;
-            D.b_trans = 0;
-            D.k_per_split = LS_HIDDEN;
-            D.epi = LM_EPI_SILU_GRAD;
-            D.z_in = S.d_z[l - 1];
-            D.out_bf16 = S.d_dz[l - 1];
-            D.ldc = K;
-            LS_CHECK(this, sg_gemm(D, 1, s));
+        // mini-batch, forward, loss, and every layer's dZ
+        lm::PassParams T;
+        std::memset(&T, 0, sizeof(T));
+        T.states = S.d_states;
+        T.targets = S.d_tscaled;
+        T.fine = S.d_targets;
+        T.n_data = n_train;
+        T.seed = cfg.seed ^ 0x5DEECE66Dull;
+        T.step = step;
+        T.rows = B;
+        T.radius = cfg.radius;
+        T.freqs = S.d_freqs;
+        T.wpack = S.d_wpack;
+        T.bpack = S.d_bpack;
+        T.w_out = S.W[4];
+        T.b_out = S.b[4];
+        T.scale_p = S.scale_p;
+        T.tol = cfg.tolerance;
+        T.conf_weight = conf_w;
+        T.loss = want_loss ? S.d_loss : nullptr;
+        T.feat = S.d_feat;
+        T.dout = S.d_dout;
+        T.z = S.d_z;
+        for (int l = 0; l < 4; ++l) {
+            T.bias[l] = S.b[l];
+            T.act[l] = S.d_act[l];
+            T.dz[l] = S.d_dz[l];
         }
+        LS_CHECK(this, sg_train_pass(T, s));
         // every gradient, then Adam
         lm::GradParams G;
         std::memset(&G, 0, sizeof(G));
         for (int l = 0; l < 4; ++l) {  // dW = X^T dZ, split over the batch
             lm::GemmParams& D = G.dw[l];
-            D.A = acts[l];
+            D.A = l == 0 ? S.d_feat : S.d_act[l - 1];
             D.B = S.d_dz[l];
             D.M = kLayerK[l];
             D.N = LS_HIDDEN;
@@ -380,7 +377,7 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
         }
         G.splits = splits;
         G.rows = B;
-        G.act_top = S.d_act[4];
+        G.act_top = S.d_act[3];
         G.dout = S.d_dout;
         G.col_part = S.d_col_part;
         G.out_part = S.d_out_part;
@@ -392,7 +389,9 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
         lm::UpdateParams U;
         std::memset(&U, 0, sizeof(U));
         for (int l = 0; l < 4; ++l)
-            U.hidden[l] = lm::LayerUpdate{S.W[l], S.mW[l], S.vW[l], S.b[l], S.mb[l], S.vb[l], S.Wt[l],
+            U.hidden[l] = lm::LayerUpdate{S.W[l], S.mW[l], S.vW[l], S.b[l], S.mb[l], S.vb[l],
+                                          S.d_wpack + lm::pack_offset(l),
+                                          l > 0 ? S.d_bpack + (size_t)(l - 1) * LM_PACK_LAYER : nullptr,
                                           S.d_part + part_at[l], kLayerK[l]};
         U.w = S.W[4];
         U.m = S.mW[4];
@@ -411,6 +410,8 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
             if (!std::isfinite(last_loss)) return fail(LINON_ERR_STATE, "surrogate: training diverged (loss NaN)");
         }
     }
+    // the [N][K] copies of the trained weights, which the kernels of one layer read
+    for (int l = 0; l < 4; ++l) LS_CHECK(this, sg_transpose(S.W[l], kLayerK[l], S.Wt[l], s));
     LS_CHECK(this, hipStreamSynchronize(s));
     auto t2 = std::chrono::steady_clock::now();
 
@@ -418,8 +419,6 @@ linon_status Context::surrogate_train(const linon_surrogate_config& cfg, linon_s
     std::vector<float> err;
     st = surrogate_eval(S.d_states + 6 * (size_t)n_train, S.d_tscaled + 6 * (size_t)n_train,
                         S.d_targets + 6 * (size_t)n_train, n_hold, err);
-    if (st != LINON_OK) return st;
-    st = surrogate_pack();
     if (st != LINON_OK) return st;
     S.trained = true;
     if (stats) {
@@ -471,15 +470,14 @@ linon_status Context::surrogate_eval(const float* states, const float* targets, 
     hipStream_t s = stream;
     lm::u16* feat = nullptr;
     lm::u16 *a0 = nullptr, *a1 = nullptr;
-    float *out = nullptr, *dout = nullptr, *e = nullptr, *loss = nullptr;
+    float *out = nullptr, *e = nullptr;
     auto cleanup = [&]() {
-        for (void* p : {(void*)feat, (void*)a0, (void*)a1, (void*)out, (void*)dout, (void*)e, (void*)loss})
+        for (void* p : {(void*)feat, (void*)a0, (void*)a1, (void*)out, (void*)e})
             if (p) (void)hipFree(p);
     };
     if (dalloc(feat, (size_t)n * LS_FEATS_PAD) != hipSuccess || dalloc(a0, (size_t)n * LS_HIDDEN) != hipSuccess ||
         dalloc(a1, (size_t)n * LS_HIDDEN) != hipSuccess || dalloc(out, (size_t)n * LS_OUT) != hipSuccess ||
-        dalloc(dout, (size_t)n * LS_OUT) != hipSuccess || dalloc(e, (size_t)n) != hipSuccess ||
-        dalloc(loss, 1) != hipSuccess) {
+        dalloc(e, (size_t)n) != hipSuccess) {
         cleanup();
         return fail(LINON_ERR_HIP, "surrogate_eval: out of device memory");
     }
@@ -488,12 +486,11 @@ linon_status Context::surrogate_eval(const float* states, const float* targets, 
         ls::SurrogateIO io{states, n, S.cfg.radius, S.d_freqs, feat};
         if (sg_features(io, s) != hipSuccess) { st = fail(LINON_ERR_HIP, "eval features"); break; }
         lm::u16* const acts[5] = {feat, a0, a1, a0, a1};
-        st = surrogate_forward(n, feat, acts, nullptr, s);
+        st = surrogate_forward(n, feat, acts, s);
         if (st != LINON_OK) break;
         if (sg_out_layer(a1, S.W[4], S.b[4], n, out, s) != hipSuccess) { st = fail(LINON_ERR_HIP, "eval out"); break; }
-        if (hipMemsetAsync(loss, 0, 4, s) != hipSuccess ||
-            sg_loss(out, targets, fine, n, S.scale_p, S.cfg.tolerance, 0.1f, dout, e, loss, s) != hipSuccess) {
-            st = fail(LINON_ERR_HIP, "eval loss");
+        if (sg_errors(out, targets, fine, n, S.scale_p, e, s) != hipSuccess) {
+            st = fail(LINON_ERR_HIP, "eval errors");
             break;
         }
         err.resize(n);

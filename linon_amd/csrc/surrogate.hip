@@ -10,6 +10,7 @@
 #include "device/mlp_fused.hpp"
 #include "device/surrogate.hpp"
 #include "device/train.hpp"
+#include "device/train_pass.hpp"
 #include "surrogate_kernels.hpp"
 
 namespace LINON_KERNEL_NS {
@@ -21,11 +22,16 @@ __global__ void __launch_bounds__(256) gemm_nt_kernel(lm::GemmParams P) { lm::ge
 __global__ void __launch_bounds__(256) gemm_tn_kernel(lm::GemmParams P) {
     lm::gemm_tn_body(P, lm::gemm_tn_work((int)blockIdx.x, (int)gridDim.x));
 }
+// two 128-row workgroups per CU (80 KB of LDS each)
+__global__ void __launch_bounds__(256, 2) train_pass_kernel(lm::PassParams P) { lm::train_pass_body(P); }
 __global__ void __launch_bounds__(256) grads_kernel(lm::GradParams P) { lm::grads_body(P); }
 __global__ void __launch_bounds__(LM_SUM_ROWS) update_kernel(lm::UpdateParams P) { lm::update_body(P); }
 
 __global__ void __launch_bounds__(256) features_kernel(ls::SurrogateIO S) { ls::features_body(S); }
-__global__ void __launch_bounds__(256) mlp_pack_kernel(const float* W, int K, u16* dst) { lm::mlp_pack_body(W, K, dst); }
+template <bool Transposed>
+__global__ void __launch_bounds__(256) mlp_pack_kernel(const float* W, int K, u16* dst) {
+    lm::mlp_pack_body<Transposed>(W, K, dst);
+}
 // two 128-ray workgroups per CU (75 KB of LDS each)
 __global__ void __launch_bounds__(256, 2) mlp_infer_kernel(lm::MlpInferParams P) { lm::mlp_infer_body(P); }
 
@@ -120,35 +126,6 @@ __global__ void __launch_bounds__(256) residual_sumsq_kernel(const float* fine, 
     }
 }
 
-// Gathers a mini-batch: rows idx[i] of the training states, network targets and RK4 exits (idx
-// from a counter-based hash of (seed, step, i)).
-__global__ void __launch_bounds__(256) gather_batch_kernel(const float* states, const float* targets,
-                                                           const float* fine, int n_data, unsigned long long seed,
-                                                           int step, int batch, float* bstates, float* btargets,
-                                                           float* bfine) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= batch) return;
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * ((unsigned long long)step * (unsigned long long)batch + i + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    const int r = (int)(z % (unsigned long long)n_data);
-    for (int k = 0; k < 6; ++k) {
-        bstates[6 * (size_t)i + k] = states[6 * (size_t)r + k];
-        btargets[6 * (size_t)i + k] = targets[6 * (size_t)r + k];
-        bfine[6 * (size_t)i + k] = fine[6 * (size_t)r + k];
-    }
-}
-
-// Exit-point error of a prediction against the RK4 exit, as the parity tests measure it:
-// max over x, y, z of |pred - exit| / max(1, |exit|).
-__device__ __forceinline__ float exit_error(float px, float py, float pz, const float* e) {
-    const float ex = fabsf(px - e[0]) / fmaxf(1.0f, fabsf(e[0]));
-    const float ey = fabsf(py - e[1]) / fmaxf(1.0f, fabsf(e[1]));
-    const float ez = fabsf(pz - e[2]) / fmaxf(1.0f, fabsf(e[2]));
-    return fmaxf(ex, fmaxf(ey, ez));
-}
-
 // FP32 output layer: out[i][o] = sum_k act[i][k] * W[k][o] + b[o] (bf16 activations, fp32
 // weights), one lane per (row, output).
 __global__ void __launch_bounds__(256) out_layer_kernel(const u16* act, const float* W, const float* b, int n,
@@ -162,54 +139,23 @@ __global__ void __launch_bounds__(256) out_layer_kernel(const u16* act, const fl
     out[(size_t)i * LS_OUT + o] = s;
 }
 
-// Loss and output gradient.  Regression: mean squared error of the 6 scaled targets.
-// Confidence: logistic loss against the label [exit-point error <= tol], the error being the
-// prediction's (base + output / scale_p) against the RK4 exit `fine`.  Writes dOut [n][LS_OUT]
-// (already / n) and the per-row error.
-__global__ void __launch_bounds__(256) loss_kernel(const float* out, const float* target, const float* fine, int n,
-                                                   float scale_p, float tol, float conf_weight, float* dout,
-                                                   float* err, float* loss_sum) {
+// Exit-point error of every row's prediction (base + output / scale_p) against its RK4 exit.
+__global__ void __launch_bounds__(256) errors_kernel(const float* out, const float* target, const float* fine, int n,
+                                                     float scale_p, float* err) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.0f;
-    if (i < n) {
-        const float* o = out + (size_t)i * LS_OUT;
-        const float* y = target + 6 * (size_t)i;
-        const float* f = fine + 6 * (size_t)i;
-        float pe[3];
-        for (int k = 0; k < 6; ++k) {
-            float d = o[k] - y[k];
-            l += d * d / 6.0f;
-            dout[(size_t)i * LS_OUT + k] = 2.0f * d / (6.0f * n);
-            if (k < 3) pe[k] = f[k] + d / scale_p;  // the prediction: exit + (output - target) / scale
-        }
-        const float e = exit_error(pe[0], pe[1], pe[2], f);
-        err[i] = e;
-        const float label = e <= tol ? 1.0f : 0.0f;
-        const float c = o[6];
-        const float s = 1.0f / (1.0f + __expf(-c));
-        l += conf_weight * (fmaxf(c, 0.0f) - c * label + log1pf(__expf(-fabsf(c))));
-        dout[(size_t)i * LS_OUT + 6] = conf_weight * (s - label) / n;
-    }
-    // block reduction of the loss
-    __shared__ float red[256];
-    red[threadIdx.x] = l;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(loss_sum, red[0] / n);
+    if (i >= n) return;
+    const float* f = fine + 6 * (size_t)i;
+    float pe[3];
+    for (int k = 0; k < 3; ++k) pe[k] = f[k] + (out[(size_t)i * LS_OUT + k] - target[6 * (size_t)i + k]) / scale_p;
+    err[i] = lm::exit_error(pe[0], pe[1], pe[2], f);
 }
 
-// Output-layer backward: dA[i][k] = sum_o dOut[i][o] W[k][o], gated by silu'(z) -> bf16 dZ.
-__global__ void __launch_bounds__(256) out_layer_back_kernel(const float* dout, const float* W, const float* z, int n,
-                                                             u16* dz) {
+// The BF16 copy [N][K] of a hidden layer's weights W [K][N], N = 256.
+__global__ void __launch_bounds__(256) transpose_kernel(const float* W, int K, u16* wt) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * LS_HIDDEN) return;
-    const int i = t / LS_HIDDEN, k = t % LS_HIDDEN;
-    float s = 0.0f;
-    for (int o = 0; o < LS_OUT; ++o) s = __builtin_fmaf(dout[(size_t)i * LS_OUT + o], W[k * LS_OUT + o], s);
-    dz[t] = lm::f2bf(s * lm::silu_grad(z[t]));
+    if (t >= K * LS_HIDDEN) return;
+    const int n = t / K, k = t % K;
+    wt[t] = lm::f2bf(W[(size_t)k * LS_HIDDEN + n]);
 }
 
 // Sums split-K partials: out[j] = sum_s part[s][j].
@@ -288,7 +234,7 @@ __global__ void __launch_bounds__(256) apply_rk4_kernel(const int* list, int n, 
     const int r = list[i];
     const float* e = exits + 6 * (size_t)r;
     if (err_out)
-        err_out[i] = exit_error(pred_exit[3 * (size_t)r], pred_exit[3 * (size_t)r + 1], pred_exit[3 * (size_t)r + 2], e);
+        err_out[i] = lm::exit_error(pred_exit[3 * (size_t)r], pred_exit[3 * (size_t)r + 1], pred_exit[3 * (size_t)r + 2], e);
     if (write_mapping) reinterpret_cast<float4*>(mapping)[texel_of[r]] = make_float4(e[0], e[1], e[2], 1.0f);
 }
 
@@ -339,8 +285,11 @@ hipError_t sg_gemm(const lm::GemmParams& P, int splits, hipStream_t s) {
 
 #define LS_GRID(n) dim3(((n) + 255) / 256), dim3(256)
 
-hipError_t sg_mlp_pack(const float* W, int K, u16* dst, hipStream_t s) {
-    hipLaunchKernelGGL(mlp_pack_kernel, LS_GRID((K / 16) * 8 * 64), 0, s, W, K, dst);
+hipError_t sg_mlp_pack(const float* W, int K, u16* dst, bool transposed, hipStream_t s) {
+    if (transposed)
+        hipLaunchKernelGGL(mlp_pack_kernel<true>, LS_GRID((K / 16) * 8 * 64), 0, s, W, K, dst);
+    else
+        hipLaunchKernelGGL(mlp_pack_kernel<false>, LS_GRID((K / 16) * 8 * 64), 0, s, W, K, dst);
     return hipGetLastError();
 }
 hipError_t sg_mlp_infer(const lm::MlpInferParams& P, hipStream_t s) {
@@ -361,24 +310,21 @@ hipError_t sg_residual_sumsq(const float* fine, const float* base, int n, float*
     hipLaunchKernelGGL(residual_sumsq_kernel, LS_GRID(n), 0, s, fine, base, n, acc);
     return hipGetLastError();
 }
-hipError_t sg_gather(const float* states, const float* targets, const float* fine, int n_data, unsigned long long seed,
-                     int step, int batch, float* bstates, float* btargets, float* bfine, hipStream_t s) {
-    hipLaunchKernelGGL(gather_batch_kernel, LS_GRID(batch), 0, s, states, targets, fine, n_data, seed, step, batch,
-                       bstates, btargets, bfine);
+hipError_t sg_train_pass(const lm::PassParams& P, hipStream_t s) {
+    hipLaunchKernelGGL(train_pass_kernel, dim3((P.rows + LM_FUSED_ROWS - 1) / LM_FUSED_ROWS), dim3(256), 0, s, P);
+    return hipGetLastError();
+}
+hipError_t sg_transpose(const float* W, int K, u16* wt, hipStream_t s) {
+    hipLaunchKernelGGL(transpose_kernel, LS_GRID(K * LS_HIDDEN), 0, s, W, K, wt);
+    return hipGetLastError();
+}
+hipError_t sg_errors(const float* out, const float* target, const float* fine, int n, float scale_p, float* err,
+                     hipStream_t s) {
+    hipLaunchKernelGGL(errors_kernel, LS_GRID(n), 0, s, out, target, fine, n, scale_p, err);
     return hipGetLastError();
 }
 hipError_t sg_out_layer(const u16* act, const float* W, const float* b, int n, float* out, hipStream_t s) {
     hipLaunchKernelGGL(out_layer_kernel, LS_GRID(n * LS_OUT), 0, s, act, W, b, n, out);
-    return hipGetLastError();
-}
-hipError_t sg_loss(const float* out, const float* target, const float* fine, int n, float scale_p, float tol,
-                   float conf_weight, float* dout, float* err, float* loss_sum, hipStream_t s) {
-    hipLaunchKernelGGL(loss_kernel, LS_GRID(n), 0, s, out, target, fine, n, scale_p, tol, conf_weight, dout, err,
-                       loss_sum);
-    return hipGetLastError();
-}
-hipError_t sg_out_layer_back(const float* dout, const float* W, const float* z, int n, u16* dz, hipStream_t s) {
-    hipLaunchKernelGGL(out_layer_back_kernel, LS_GRID(n * LS_HIDDEN), 0, s, dout, W, z, n, dz);
     return hipGetLastError();
 }
 hipError_t sg_reduce(const float* part, int splits, int n, float* out, hipStream_t s) {

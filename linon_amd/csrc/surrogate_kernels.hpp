@@ -6,6 +6,7 @@
 #include "device/mlp_fused.hpp"
 #include "device/surrogate.hpp"
 #include "device/train.hpp"
+#include "device/train_pass.hpp"
 
 // Compiled twice like kernels.hip: LINON_KERNEL_NS is linon (IEEE) or linon_wgslmath (WGSL
 // accuracy); the RK4 legs of a surrogate frame use the build the plain kernel of that field uses.
@@ -17,18 +18,16 @@
     bool sg_field_supported(int field); \
     hipError_t sg_gemm(const lm::GemmParams& P, int splits, hipStream_t s); \
     hipError_t sg_features(const ls::SurrogateIO& S, hipStream_t s); \
-    hipError_t sg_mlp_pack(const float* W, int K, lm::u16* dst, hipStream_t s); \
+    hipError_t sg_mlp_pack(const float* W, int K, lm::u16* dst, bool transposed, hipStream_t s); \
     hipError_t sg_mlp_infer(const lm::MlpInferParams& P, hipStream_t s); \
     hipError_t sg_make_targets(const float* fine, const float* base, int n, float scale_p, float scale_d, float* tgt, \
                                hipStream_t s); \
     hipError_t sg_residual_sumsq(const float* fine, const float* base, int n, float* acc, hipStream_t s); \
-    hipError_t sg_gather(const float* states, const float* targets, const float* fine, int n_data, \
-                         unsigned long long seed, int step, int batch, float* bstates, float* btargets, float* bfine, \
+    hipError_t sg_train_pass(const lm::PassParams& P, hipStream_t s); \
+    hipError_t sg_transpose(const float* W, int K, lm::u16* wt, hipStream_t s); \
+    hipError_t sg_errors(const float* out, const float* target, const float* fine, int n, float scale_p, float* err, \
                          hipStream_t s); \
     hipError_t sg_out_layer(const lm::u16* act, const float* W, const float* b, int n, float* out, hipStream_t s); \
-    hipError_t sg_loss(const float* out, const float* target, const float* fine, int n, float scale_p, float tol, \
-                       float conf_weight, float* dout, float* err, float* loss_sum, hipStream_t s); \
-    hipError_t sg_out_layer_back(const float* dout, const float* W, const float* z, int n, lm::u16* dz, hipStream_t s); \
     hipError_t sg_reduce(const float* part, int splits, int n, float* out, hipStream_t s); \
     hipError_t sg_grads(const lm::GradParams& P, hipStream_t s); \
     hipError_t sg_update(const lm::UpdateParams& P, hipStream_t s); \
