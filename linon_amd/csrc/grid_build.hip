@@ -1,17 +1,23 @@
 // Device build of the uniform grid (the host build in grid.cpp computes the same arrays):
-//   1. count: one lane per face counts, per overlapped cell, one reference (atomic add);
-//   2. exclusive scan of the per-cell counts (64-bit, block scans + one pass over the block
-//      sums) -> cell_start;
-//   3. fill: the same overlap decisions again, each reference placed at cell_start[cell] plus
-//      an atomic cursor;
-//   4. each cell's list sorted by face id (the host build's ascending order);
-//   5. Chebyshev distance field: a 1-D distance along x, then min-max passes along y and z.
-// The overlap test is the shared double-precision separating-axis test with contraction off,
-// so every decision, and therefore every array, equals the host build's.
+//   1. overlap: 16 lanes per face test its cells; which of them it overlaps is kept as a bit mask,
+//      how many as the face's count.  A face with more than 256 cells in range gets a wave, one
+//      with more than 8192 (a wall) is spread over the blocks;
+//   2. exclusive scan of the face counts -> where each face's references stand, and their total;
+//   3. place: every reference takes its slot in its cell (an atomic counter per cell) and is
+//      recorded as (cell, slot, face);
+//   4. exclusive scan of the cell counts -> cell_start;
+//   5. each reference goes to its cell's list, then to its rank there (how many of the list's
+//      faces have a smaller id): the host build's ascending order;
+//   6. Chebyshev distance field: the distance along x from each row's occupancy bits, then min-max
+//      passes along y and z.
+// The overlap decisions are those of the shared double-precision separating-axis test with
+// contraction off (FaceTest below settles nearly all of them with a fraction of its arithmetic),
+// so every array equals the host build's.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <string>
+#include <vector>
 
 #include "device/grid_sat.hpp"
 #include "grid_build.hpp"
@@ -29,82 +35,309 @@ __device__ __forceinline__ void load_face(const float* xyz, const uint32_t* face
     }
 }
 
-// Faces whose cell range holds more than this many cells are tested cell-parallel by a whole
-// block (grid_cells_big_kernel) instead of by one lane: a wall of the Cornell box spans 2 x 256^2
-// cells of the 256^3 grid, against a handful for an icosphere face.
-constexpr size_t kBigFaceCells = 256;
+// Faces whose cell range holds more than kMidFaceCells cells are tested by a wave each, those with
+// more than kHugeFaceCells by many blocks: a wall of the Cornell box spans 3 x 256^2 cells of the
+// 256^3 grid, a face of a displaced icosphere a handful to a few hundred.  Above 8192 cells a lone
+// wave becomes the launch's tail (the Cornell box's inner faces in 128^3 cells: 97 us with the line
+// at 16384, 16 us with it at 2048), while faces spread over blocks cost each block the face's set-up
+// (1.3 M faces, many of 2048 to 8192 cells in 256^3: 3.2 ms with the line at 2048).
+constexpr size_t kMidFaceCells = 256, kHugeFaceCells = 8192;
+
+constexpr int kFaceLanes = 16;  // lanes per face in the overlap test: 16 cells a lane at most
+static_assert(kMidFaceCells == (size_t)kFaceLanes * 16, "a lane's cells fill a 16-bit mask");
 
 __device__ __forceinline__ size_t range_cells(const int c0[3], const int c1[3]) {
     return (size_t)(c1[0] - c0[0] + 1) * (size_t)(c1[1] - c0[1] + 1) * (size_t)(c1[2] - c0[2] + 1);
 }
 
-// One reference of face f to cell (x, y, z): count it (FILL = false) or place it (FILL = true).
-template <bool FILL>
-__device__ __forceinline__ void add_reference(const GridGeom& g, size_t f, int x, int y, int z, unsigned* counter,
-                                              const unsigned* cell_start, unsigned* cell_faces, unsigned* overflow) {
-    const size_t cell = ((size_t)z * (size_t)g.dim[1] + (size_t)y) * (size_t)g.dim[0] + (size_t)x;
-    if (!FILL) {
-        atomicAdd(counter + cell, 1u);
-    } else {
-        const unsigned slot = atomicAdd(counter + cell, 1u);
-        const unsigned b = cell_start[cell], e = cell_start[cell + 1];
-        if (slot < e - b)
-            cell_faces[b + slot] = (unsigned)f;
-        else
-            atomicOr(overflow, 1u);  // counts and placements disagree: reported, never written
+// Cell k of a face's range, x fastest.  At most 1024^3 cells, so 32 bits hold every index.
+struct FaceCells {
+    int x0, y0, z0;
+    unsigned sx, sxy;
+    __device__ __forceinline__ FaceCells(const int c0[3], const int c1[3])
+        : x0(c0[0]), y0(c0[1]), z0(c0[2]), sx((unsigned)(c1[0] - c0[0] + 1)),
+          sxy(sx * (unsigned)(c1[1] - c0[1] + 1)) {}
+    __device__ __forceinline__ void at(unsigned k, int& x, int& y, int& z) const {
+        const unsigned kz = k / sxy, r = k - kz * sxy, ky = r / sx;
+        x = x0 + (int)(r - ky * sx);
+        y = y0 + (int)ky;
+        z = z0 + (int)kz;
     }
+};
+
+__device__ __forceinline__ unsigned cell_index(const GridGeom& g, int x, int y, int z) {
+    return ((unsigned)z * (unsigned)g.dim[1] + (unsigned)y) * (unsigned)g.dim[0] + (unsigned)x;
 }
 
-// Count (FILL = false) or place (FILL = true) the references of one face per lane.  Faces with
-// more than kBigFaceCells cells in range are left to grid_cells_big_kernel; the counting pass
-// lists them in big[0 .. *nbig).
-template <bool FILL>
-__global__ void __launch_bounds__(256) grid_cells_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
-                                                         uint32_t nf, unsigned* counter, const unsigned* cell_start,
-                                                         unsigned* cell_faces, unsigned* overflow, unsigned* big,
-                                                         unsigned* nbig) {
+struct Reference {
+    unsigned cell, slot, face;
+};
+
+// The separating-axis test of one face with what depends on the face alone computed once: the
+// projections of the three vertices on each of the 13 axes, widened by the box's half extent.  A
+// cell is then settled by the projection of its centre, about 70 double-precision operations
+// where face_in_cell takes 350, unless some axis comes within a slack of its threshold, which
+// covers the rounding of both computations; those cells (about one in 10^11) take face_in_cell
+// itself.  With |vertices|, |centres| <= S both projections onto an edge axis are off by less than
+// 2^-46 S^2, onto the normal by less than 2^-42 S^3, and onto a box axis by 2^-50 S; the slacks are
+// 8 times that and more.  An axis that is exactly zero (an edge along it: the difference of equal
+// coordinates is zero in both computations) separates nothing and has infinite thresholds.
+struct FaceTest {
+    double e[3][3];            // edges
+    double lo[9], hi[9];       // thresholds of the edge axes (3 j + i: edge j x unit vector i)
+    double blo[3], bhi[3];     // of the box axes
+    double n[3], nlo, nhi;     // the normal and its thresholds
+    double slack_e, slack_b, slack_n;
+
+    __device__ __forceinline__ FaceTest(const GridGeom& g, const double v[3][3]) {
+        const double h = 0.5 * g.cs + g.margin;
+        double S = 0.0;
+        for (int k = 0; k < 3; ++k)
+            S = gs_max(S, gs_max(gs_abs((double)g.lo[k]), gs_abs((double)g.hi[k])));
+        S += g.cs + g.margin;  // the grid's box, which holds every vertex, and a cell more
+        slack_e = S * S * 0x1p-43;
+        slack_b = S * 0x1p-46;
+        slack_n = S * S * S * 0x1p-38;
+        for (int k = 0; k < 3; ++k) {
+            e[0][k] = v[1][k] - v[0][k];
+            e[1][k] = v[2][k] - v[1][k];
+            e[2][k] = v[0][k] - v[2][k];
+            blo[k] = gs_min(v[0][k], gs_min(v[1][k], v[2][k])) - h;
+            bhi[k] = gs_max(v[0][k], gs_max(v[1][k], v[2][k])) + h;
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double q0 = along(j, i, v[0]), q1 = along(j, i, v[1]), q2 = along(j, i, v[2]);
+                const double p = e[j][(i + 1) % 3], q = e[j][(i + 2) % 3];
+                const double r = h * (gs_abs(p) + gs_abs(q));
+                const bool none = p == 0.0 && q == 0.0;
+                lo[3 * j + i] = none ? -__builtin_inf() : gs_min(q0, gs_min(q1, q2)) - r;
+                hi[3 * j + i] = none ? __builtin_inf() : gs_max(q0, gs_max(q1, q2)) + r;
+            }
+        n[0] = e[0][1] * e[1][2] - e[0][2] * e[1][1];
+        n[1] = e[0][2] * e[1][0] - e[0][0] * e[1][2];
+        n[2] = e[0][0] * e[1][1] - e[0][1] * e[1][0];
+        const double d = n[0] * v[0][0] + n[1] * v[0][1] + n[2] * v[0][2];
+        const double r = h * (gs_abs(n[0]) + gs_abs(n[1]) + gs_abs(n[2]));
+        nlo = d - r;
+        nhi = d + r;
+    }
+    // projection on edge j x unit vector i, up to sign: e_(i+1) x_(i+2) - e_(i+2) x_(i+1)
+    __device__ __forceinline__ double along(int j, int i, const double x[3]) const {
+        const int a = (i + 1) % 3, b = (i + 2) % 3;
+        return e[j][a] * x[b] - e[j][b] * x[a];
+    }
+    __device__ __forceinline__ bool in_cell(const GridGeom& g, const double v[3][3], int x, int y, int z) const {
+        const double c[3] = {(double)g.lo[0] + (x + 0.5) * g.cs, (double)g.lo[1] + (y + 0.5) * g.cs,
+                             (double)g.lo[2] + (z + 0.5) * g.cs};
+        double ge = -__builtin_inf(), gb = -__builtin_inf();  // widest gaps
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double s = along(j, i, c);
+                ge = __builtin_fmax(ge, __builtin_fmax(lo[3 * j + i] - s, s - hi[3 * j + i]));
+            }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gb = __builtin_fmax(gb, __builtin_fmax(blo[k] - c[k], c[k] - bhi[k]));
+        const double s = n[0] * c[0] + n[1] * c[1] + n[2] * c[2];
+        const double gn = __builtin_fmax(nlo - s, s - nhi);
+        if (ge > slack_e || gb > slack_b || gn > slack_n) return false;
+        if (ge < -slack_e && gb < -slack_b && gn < -slack_n) return true;
+        return face_in_cell(g, v, x, y, z);
+    }
+};
+
+// Lists the faces that face_overlap_kernel leaves alone: mid ones from the front of big[nf], huge
+// ones from its back; nbig[2] counts them.  One atomic per class and block of 1024 faces: they all
+// go to two addresses, about 9 ns each.
+__global__ void __launch_bounds__(1024) classify_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
+                                                        uint32_t nf, unsigned* big, unsigned* nbig) {
+    __shared__ unsigned base[2][16];
     const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    size_t cells = 0;
+    if (f < nf) {
+        double v[3][3];
+        load_face(xyz, faces, (uint32_t)f, v);
+        int c0[3], c1[3];
+        face_cell_range(g, v, c0, c1);
+        if (c1[0] >= c0[0] && c1[1] >= c0[1] && c1[2] >= c0[2]) cells = range_cells(c0, c1);
+    }
+    const bool huge = cells > kHugeFaceCells, mid = cells > kMidFaceCells && !huge;
+    const unsigned long long m = __ballot(mid), h = __ballot(huge);
+    if (lane == 0) {
+        base[0][wave] = (unsigned)__popcll(m);
+        base[1][wave] = (unsigned)__popcll(h);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned* c = base[threadIdx.x];
+        unsigned n = 0;
+        for (int w = 0; w < 16; ++w) n += c[w];
+        unsigned at = n ? atomicAdd(nbig + threadIdx.x, n) : 0u;
+        for (int w = 0; w < 16; ++w) {
+            const unsigned k = c[w];
+            c[w] = at;
+            at += k;
+        }
+    }
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (mid) big[base[0][wave] + (unsigned)__popcll(m & below)] = (unsigned)f;
+    if (huge) big[nf - 1u - (base[1][wave] + (unsigned)__popcll(h & below))] = (unsigned)f;
+}
+
+// Overlap test, 16 lanes per face: lane s tests cells s, s + 16, ... of the face's range and keeps
+// bit i for cell s + 16 i.  One lane per face left a 20,516-face mesh 80 blocks, each lane testing
+// up to 256 cells one after another (0.5 ms, twice: the second time to place them).
+__global__ void __launch_bounds__(256) face_overlap_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
+                                                           uint32_t nf, unsigned short* masks, unsigned* count) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t f = t / kFaceLanes;
+    const unsigned sub = (unsigned)t % kFaceLanes;
     if (f >= nf) return;
     double v[3][3];
     load_face(xyz, faces, (uint32_t)f, v);
     int c0[3], c1[3];
     face_cell_range(g, v, c0, c1);
-    if (c1[0] < c0[0] || c1[1] < c0[1] || c1[2] < c0[2]) return;  // outside the grid (cannot happen)
-    if (range_cells(c0, c1) > kBigFaceCells) {
-        if (!FILL) big[atomicAdd(nbig, 1u)] = (unsigned)f;  // at most nf entries
-        return;
-    }
-    for (int z = c0[2]; z <= c1[2]; ++z)
-        for (int y = c0[1]; y <= c1[1]; ++y)
-            for (int x = c0[0]; x <= c1[0]; ++x)
-                if (face_in_cell(g, v, x, y, z))
-                    add_reference<FILL>(g, f, x, y, z, counter, cell_start, cell_faces, overflow);
-}
-
-// The faces listed by the counting pass, one block per face at a time (grid-stride over the
-// list), its lanes striding over the face's cell range.
-template <bool FILL>
-__global__ void __launch_bounds__(256) grid_cells_big_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
-                                                             const unsigned* big, const unsigned* nbig,
-                                                             unsigned* counter, const unsigned* cell_start,
-                                                             unsigned* cell_faces, unsigned* overflow) {
-    const unsigned n = *nbig;
-    for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
-        const size_t f = big[i];
-        double v[3][3];
-        load_face(xyz, faces, (uint32_t)f, v);
-        int c0[3], c1[3];
-        face_cell_range(g, v, c0, c1);
-        const size_t sx = (size_t)(c1[0] - c0[0] + 1), sy = (size_t)(c1[1] - c0[1] + 1);
+    unsigned mask = 0;
+    // (an empty range, outside the grid, cannot happen: the grid encloses every face)
+    if (c1[0] >= c0[0] && c1[1] >= c0[1] && c1[2] >= c0[2]) {
         const size_t cells = range_cells(c0, c1);
-        for (size_t k = threadIdx.x; k < cells; k += blockDim.x) {
-            const int x = c0[0] + (int)(k % sx);
-            const int y = c0[1] + (int)((k / sx) % sy);
-            const int z = c0[2] + (int)(k / (sx * sy));
-            if (face_in_cell(g, v, x, y, z))
-                add_reference<FILL>(g, f, x, y, z, counter, cell_start, cell_faces, overflow);
+        if (cells <= kMidFaceCells) {
+            const FaceCells C(c0, c1);
+            const FaceTest T(g, v);
+            int x, y, z;
+            for (unsigned k = sub, i = 0; k < (unsigned)cells; k += kFaceLanes, ++i) {
+                C.at(k, x, y, z);
+                if (T.in_cell(g, v, x, y, z)) mask |= 1u << i;
+            }
         }
     }
+    masks[t] = (unsigned short)mask;
+    unsigned n = (unsigned)__popc(mask);
+    for (int off = kFaceLanes / 2; off > 0; off >>= 1) n += __shfl_xor(n, off, kFaceLanes);
+    if (sub == 0) count[f] = n;  // 0 for a listed face: its own kernel adds its references
+}
+
+// A reference's slot in its cell.
+__device__ __forceinline__ Reference take_slot(unsigned cell, unsigned face, unsigned* cell_count) {
+    return Reference{cell, atomicAdd(cell_count + cell, 1u), face};
+}
+
+// The references the overlap test found, from the masks (16 lanes per face as there).
+__global__ void __launch_bounds__(256) face_place_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
+                                                         uint32_t nf, const unsigned short* masks,
+                                                         const unsigned* first, unsigned* cell_count, Reference* refs) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t f = t / kFaceLanes;
+    const unsigned sub = (unsigned)t % kFaceLanes;
+    if (f >= nf) return;
+    unsigned mask = masks[t];
+    const unsigned n = (unsigned)__popc(mask);
+    unsigned upto = n;  // inclusive prefix over the face's lanes
+    for (unsigned off = 1; off < (unsigned)kFaceLanes; off <<= 1) {
+        const unsigned x = __shfl_up(upto, off, kFaceLanes);
+        if (sub >= off) upto += x;
+    }
+    if (!mask) return;
+    double v[3][3];
+    load_face(xyz, faces, (uint32_t)f, v);
+    int c0[3], c1[3];
+    face_cell_range(g, v, c0, c1);
+    const FaceCells C(c0, c1);
+    Reference* out = refs + first[f] + (upto - n);
+    int x, y, z;
+    for (; mask; mask &= mask - 1) {
+        C.at(sub + kFaceLanes * (unsigned)(__ffs((int)mask) - 1), x, y, z);
+        *out++ = take_slot(cell_index(g, x, y, z), (unsigned)f, cell_count);
+    }
+}
+
+// The mid faces, a wave each (grid-stride over the list), or, with Huge, the huge ones:
+// blockIdx.x strides over the faces, the lanes of all blockIdx.y over a face's cell range.  Count
+// (PLACE = false), or place the references of a face from first[face] on: a wave that has its face
+// to itself counts along, the blocks of a huge one share a cursor.  (One block per face took 6.3 ms
+// for 1.3 M displaced-icosphere faces and the Cornell box in 256^3 cells, most of it in the 12
+// walls.)
+template <bool Huge, bool PLACE>
+__global__ void __launch_bounds__(256) big_overlap_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
+                                                          uint32_t nf, const unsigned* big, const unsigned* nbig,
+                                                          unsigned* count, const unsigned* first, unsigned* cursor,
+                                                          unsigned* cell_count, Reference* refs) {
+    const unsigned n = nbig[Huge ? 1 : 0];
+    const unsigned lane = threadIdx.x & 63;
+    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned begin = Huge ? blockIdx.x : blockIdx.x * 4 + wave;
+    const unsigned stride = Huge ? gridDim.x : gridDim.x * 4;
+    for (unsigned i = begin; i < n; i += stride) {
+        const unsigned f = big[Huge ? nf - 1u - i : i];
+        double v[3][3];
+        load_face(xyz, faces, f, v);
+        int c0[3], c1[3];
+        face_cell_range(g, v, c0, c1);
+        const FaceCells C(c0, c1);
+        const FaceTest T(g, v);
+        const unsigned cells = (unsigned)range_cells(c0, c1);
+        unsigned found = 0;
+        // 64 neighbouring cells at a time, so that a wave's lanes stay together for the ballot
+        const unsigned k_begin = Huge ? (blockIdx.y * 4 + wave) * 64 : 0, k_stride = Huge ? gridDim.y * 256 : 64;
+        for (unsigned k0 = k_begin; k0 < cells; k0 += k_stride) {
+            const unsigned k = k0 + lane;
+            int x = 0, y = 0, z = 0;
+            bool in = k < cells;
+            if (in) {
+                C.at(k, x, y, z);
+                in = T.in_cell(g, v, x, y, z);
+            }
+            const unsigned long long lanes = __ballot(in);
+            if (!lanes) continue;
+            if (PLACE) {
+                unsigned base = found;
+                if (Huge) {
+                    if (lane == 0) base = atomicAdd(cursor + i, (unsigned)__popcll(lanes));
+                    base = __shfl(base, 0, 64);
+                }
+                if (in)
+                    refs[(size_t)first[f] + base + (unsigned)__popcll(lanes & ((1ull << lane) - 1ull))] =
+                        take_slot(cell_index(g, x, y, z), f, cell_count);
+            }
+            found += (unsigned)__popcll(lanes);
+        }
+        if (!PLACE && lane == 0) {
+            if (!Huge)
+                count[f] = found;
+            else if (found)
+                atomicAdd(count + f, found);
+        }
+    }
+}
+
+// Each reference to its slot of its cell's list.
+__global__ void __launch_bounds__(256) list_kernel(const Reference* refs, size_t n, const unsigned* cell_start,
+                                                   unsigned* list) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const Reference r = refs[i];
+    list[(size_t)cell_start[r.cell] + r.slot] = r.face;
+}
+
+// Each reference to its rank in its cell: the ascending order of the face ids (distinct in a
+// cell).  A lane compares against its cell's whole list, so a list of L faces takes L^2
+// comparisons side by side, where an insertion sort by one lane takes as many in a chain (0.9 ms
+// for 1.3 M faces in 256^3 cells).
+__global__ void __launch_bounds__(256) rank_kernel(const Reference* refs, size_t n, const unsigned* cell_start,
+                                                   const unsigned* list, unsigned* cell_faces) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const Reference r = refs[i];
+    const unsigned b = cell_start[r.cell], e = cell_start[r.cell + 1];
+    unsigned rank = 0;
+    for (unsigned j = b; j < e; ++j) rank += list[j] < r.face ? 1u : 0u;
+    cell_faces[(size_t)b + rank] = r.face;
 }
 
 __device__ __forceinline__ unsigned long long block_inclusive_scan(unsigned long long v, unsigned long long* s) {
@@ -169,73 +402,76 @@ __global__ void __launch_bounds__(256) fill_u32_kernel(unsigned* p, size_t n, un
     if (i < n) p[i] = value;
 }
 
-// Ascending face ids inside every cell (lists are short; insertion sort per lane).
-__global__ void __launch_bounds__(256) sort_cells_kernel(const unsigned* cell_start, size_t nc, unsigned* faces) {
-    const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    const unsigned b = cell_start[c], e = cell_start[c + 1];
-    for (unsigned i = b + 1; i < e; ++i) {
-        const unsigned key = faces[i];
-        unsigned j = i;
-        while (j > b && faces[j - 1] > key) {
-            faces[j] = faces[j - 1];
-            --j;
-        }
-        faces[j] = key;
-    }
-}
+constexpr int kRowChunks = 1024 / 64;  // 64-cell chunks of the longest row
 
-// Distance along x to the nearest occupied cell of the row (capped at 255): a forward and a
-// backward sweep per row.
+// Distance along x to the nearest occupied cell of the row (capped at 255), one wave per row: the
+// row's occupancy as 64-bit masks, in which every lane finds the nearest set bit on either side.
+// (A sweep of each row by one lane took 76 us for 128^3 cells, 374 us for 256^3.)
 __global__ void __launch_bounds__(256) dist_x_kernel(const unsigned* cell_start, int nx, size_t rows,
                                                      unsigned char* a) {
-    const size_t row = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
+    __shared__ unsigned long long bits[4][kRowChunks];
+    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const size_t row = (size_t)blockIdx.x * 4 + wave;
+    const bool in = row < rows;
     const size_t base = row * (size_t)nx;
-    int d = 255;
-    for (int x = 0; x < nx; ++x) {
-        const bool occ = cell_start[base + x + 1] > cell_start[base + x];
-        d = occ ? 0 : (d + 1 < 255 ? d + 1 : 255);
-        a[base + x] = (unsigned char)d;
+    const int chunks = (nx + 63) / 64;
+    for (int c = 0; c < chunks; ++c) {
+        const int x = 64 * c + lane;
+        const bool occ = in && x < nx && cell_start[base + x + 1] > cell_start[base + x];
+        const unsigned long long m = __ballot(occ);
+        if (lane == 0) bits[wave][c] = m;
     }
-    d = 255;
-    for (int x = nx - 1; x >= 0; --x) {
-        d = a[base + x] == 0 ? 0 : (d + 1 < 255 ? d + 1 : 255);
-        if (d < a[base + x]) a[base + x] = (unsigned char)d;
+    __syncthreads();
+    if (!in) return;
+    for (int c = 0; c < chunks; ++c) {
+        const int x = 64 * c + lane;
+        if (x >= nx) break;
+        int d = 255;
+        // left, the cell itself included: the highest set bit at or below it
+        unsigned long long m = bits[wave][c] & (~0ull >> (63 - lane));
+        for (int k = c;;) {
+            if (m) {
+                d = min(d, x - (64 * k + 63 - __clzll((long long)m)));
+                break;
+            }
+            if (--k < 0 || x - (64 * k + 63) >= 255) break;
+            m = bits[wave][k];
+        }
+        // right: the lowest set bit at or above it
+        m = bits[wave][c] & (~0ull << lane);
+        for (int k = c;;) {
+            if (m) {
+                d = min(d, 64 * k + __ffsll((long long)m) - 1 - x);
+                break;
+            }
+            if (++k >= chunks || 64 * k - x >= 255) break;
+            m = bits[wave][k];
+        }
+        a[base + x] = (unsigned char)d;
     }
 }
 
-// out[i] = min over j of max(|i - j|, in[j]) along one line (n samples, stride s), searched
-// outwards from i until the offset alone reaches the best value.  y lines: line = (z, x);
-// z lines: line = (y, x).
+// out[i] = min over j of max(|i - j|, in[j]) along y (axis 1) or z (axis 2), one lane per cell,
+// searched outwards from i until the offset alone reaches the best value.  Neighbouring lanes are
+// neighbours in x, so every load of the search is coalesced.  (One lane per line, 16,384 of them
+// for 128^3 cells, took 418 us a pass, 1.7 ms for 256^3.)
 __global__ void __launch_bounds__(256) dist_minmax_kernel(const unsigned char* in, unsigned char* out, int nx,
                                                           int ny, int nz, int axis) {
-    const size_t line = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t base, s;
-    int n;
-    if (axis == 1) {
-        if (line >= (size_t)nz * nx) return;
-        base = (line / nx) * (size_t)nx * ny + line % nx;
-        s = (size_t)nx;
-        n = ny;
-    } else {
-        if (line >= (size_t)ny * nx) return;
-        base = line;
-        s = (size_t)nx * ny;
-        n = nz;
+    const size_t cell = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell >= (size_t)nx * ny * nz) return;
+    const unsigned row = (unsigned)cell / (unsigned)nx;  // at most 2^30 cells
+    const int i = (int)(axis == 1 ? row % (unsigned)ny : row / (unsigned)ny);
+    const int n = axis == 1 ? ny : nz;
+    const size_t s = axis == 1 ? (size_t)nx : (size_t)nx * ny;
+    const unsigned char* p = in + cell;
+    int best = *p;
+    for (int dlt = 1; dlt < best; ++dlt) {
+        int g = 255;
+        if (i - dlt >= 0) g = min(g, (int)p[-(ptrdiff_t)((size_t)dlt * s)]);
+        if (i + dlt < n) g = min(g, (int)p[(size_t)dlt * s]);
+        best = min(best, max(dlt, g));
     }
-    const unsigned char* src = in + base;
-    unsigned char* dst = out + base;
-    for (int i = 0; i < n; ++i) {
-        int best = src[(size_t)i * s];
-        for (int dlt = 1; dlt < best; ++dlt) {
-            int g = 255;
-            if (i - dlt >= 0) g = min(g, (int)src[(size_t)(i - dlt) * s]);
-            if (i + dlt < n) g = min(g, (int)src[(size_t)(i + dlt) * s]);
-            best = min(best, max(dlt, g));
-        }
-        dst[(size_t)i * s] = (unsigned char)best;
-    }
+    out[cell] = (unsigned char)best;
 }
 
 // Per-face (v0, v1 - v0, v2 - v0) as three float4 (f32 subtraction, as the shader's edges).
@@ -263,102 +499,142 @@ void DeviceGrid::release() {
     refs = 0;
 }
 
+namespace {
+
+// A sequence of arrays in one allocation, each 256-byte aligned: declare them, allocate, then ask
+// for the pointers in the same order.
+struct Arena {
+    std::vector<size_t> at;
+    size_t bytes = 0;
+    char* base = nullptr;
+    template <class T>
+    int add(size_t n) {
+        at.push_back(bytes);
+        bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+        return (int)at.size() - 1;
+    }
+    hipError_t allocate() { return hipMalloc(&base, bytes); }
+    template <class T>
+    T* get(int i) const {
+        return reinterpret_cast<T*>(base + at[(size_t)i]);
+    }
+    ~Arena() {
+        if (base) (void)hipFree(base);
+    }
+};
+
+}  // namespace
+
 bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
                        hipStream_t s, DeviceGrid& out, std::string& err) {
     out.release();
     const size_t nx = (size_t)g.dim[0], ny = (size_t)g.dim[1], nz = (size_t)g.dim[2];
     const size_t nc = nx * ny * nz;
-    const size_t nb = (nc + kScanBlock - 1) / kScanBlock;
-    float* d_xyz = nullptr;
-    uint32_t* d_faces = nullptr;
-    unsigned* d_count = nullptr;
-    unsigned long long *d_local = nullptr, *d_bsum = nullptr, *d_total = nullptr;
-    unsigned* d_flag = nullptr;
-    unsigned* d_big = nullptr;   // faces left to the block-per-face kernel, and their count
-    unsigned* d_nbig = nullptr;
-    unsigned char* d_tmp = nullptr;
-    bool ok = false;
+    const size_t longest = std::max<size_t>(nc, nf);
+    const size_t max_blocks = (longest + kScanBlock - 1) / kScanBlock;
+    Arena A, R;
+    const int i_xyz = A.add<float>(3 * (size_t)nv), i_faces = A.add<uint32_t>(3 * (size_t)nf);
+    const int i_masks = A.add<unsigned short>((size_t)nf * kFaceLanes);
+    const int i_count = A.add<unsigned>(nf), i_first = A.add<unsigned>(nf), i_big = A.add<unsigned>(nf);
+    const int i_cursor = A.add<unsigned>(nf), i_cells = A.add<unsigned>(nc);
+    const int i_local = A.add<unsigned long long>(longest), i_bsum = A.add<unsigned long long>(max_blocks);
+    const int i_total = A.add<unsigned long long>(1), i_nbig = A.add<unsigned>(2), i_tmp = A.add<unsigned char>(nc);
     auto check = [&](hipError_t e, const char* what) {
         if (e != hipSuccess) err = std::string("device grid build: ") + what + ": " + hipGetErrorString(e);
         return e == hipSuccess;
     };
-    do {
-        if (!check(hipMalloc(&d_xyz, std::max<size_t>(1, 3 * (size_t)nv) * 4), "alloc") ||
-            !check(hipMalloc(&d_faces, std::max<size_t>(1, 3 * (size_t)nf) * 4), "alloc") ||
-            !check(hipMalloc(&d_count, nc * 4), "alloc") || !check(hipMalloc(&d_local, nc * 8), "alloc") ||
-            !check(hipMalloc(&d_bsum, nb * 8), "alloc") || !check(hipMalloc(&d_total, 8), "alloc") ||
-            !check(hipMalloc(&d_flag, 4), "alloc") || !check(hipMalloc(&d_tmp, nc), "alloc") ||
-            !check(hipMalloc(&d_big, std::max<size_t>(1, (size_t)nf) * 4), "alloc") ||
-            !check(hipMalloc(&d_nbig, 4), "alloc") ||
-            !check(hipMalloc(&out.cell_start, (nc + 1) * 4), "alloc") || !check(hipMalloc(&out.dist, nc), "alloc") ||
+    auto build = [&]() {
+        if (!check(A.allocate(), "alloc") || !check(hipMalloc(&out.cell_start, (nc + 1) * 4), "alloc") ||
+            !check(hipMalloc(&out.dist, nc), "alloc") ||
             !check(hipMalloc(&out.tris, std::max<size_t>(1, (size_t)nf) * 48), "alloc"))
-            break;
-        if (nv && !check(hipMemcpyAsync(d_xyz, h_xyz, 3 * (size_t)nv * 4, hipMemcpyHostToDevice, s), "upload")) break;
-        if (nf && !check(hipMemcpyAsync(d_faces, h_faces, 3 * (size_t)nf * 4, hipMemcpyHostToDevice, s), "upload"))
-            break;
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s, d_count, nc, 0u);
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, d_flag, (size_t)1, 0u);
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, d_nbig, (size_t)1, 0u);
-        const unsigned big_blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(nf, 8192));
+            return false;
+        float* d_xyz = A.get<float>(i_xyz);
+        uint32_t* d_faces = A.get<uint32_t>(i_faces);
+        unsigned short* d_masks = A.get<unsigned short>(i_masks);
+        unsigned *d_count = A.get<unsigned>(i_count), *d_first = A.get<unsigned>(i_first);
+        unsigned *d_big = A.get<unsigned>(i_big), *d_nbig = A.get<unsigned>(i_nbig);
+        unsigned *d_cursor = A.get<unsigned>(i_cursor), *d_cells = A.get<unsigned>(i_cells);
+        unsigned long long *d_local = A.get<unsigned long long>(i_local), *d_bsum = A.get<unsigned long long>(i_bsum);
+        unsigned long long* d_total = A.get<unsigned long long>(i_total);
+        unsigned char* d_tmp = A.get<unsigned char>(i_tmp);
+        // exclusive scan of n counts into `to`, their total into d_total
+        auto scan = [&](const unsigned* counts, size_t n, unsigned* to) {
+            const size_t nb = (n + kScanBlock - 1) / kScanBlock;
+            hipLaunchKernelGGL(scan_local_kernel, dim3((unsigned)nb), dim3(256), 0, s, counts, n, d_local, d_bsum);
+            hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, s, d_bsum, nb, d_total);
+            hipLaunchKernelGGL(scan_finish_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, d_local, d_bsum, n, to);
+        };
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s, d_cells, nc, 0u);
+        unsigned long long total = 0;
+        const dim3 mid_grid((unsigned)std::max<size_t>(1, std::min<size_t>(((size_t)nf + 3) / 4, 4096)));
+        const dim3 huge_grid((unsigned)std::max<size_t>(1, std::min<size_t>(nf, 64)), 64);
+        const unsigned face_blocks = blocks_for((size_t)nf * kFaceLanes, 256);
         if (nf) {
-            hipLaunchKernelGGL(grid_cells_kernel<false>, dim3(blocks_for(nf, 256)), dim3(256), 0, s, g, d_xyz,
-                               d_faces, nf, d_count, (const unsigned*)nullptr, (unsigned*)nullptr, d_flag, d_big,
-                               d_nbig);
-            hipLaunchKernelGGL(grid_cells_big_kernel<false>, dim3(big_blocks), dim3(256), 0, s, g, d_xyz, d_faces,
-                               (const unsigned*)d_big, (const unsigned*)d_nbig, d_count, (const unsigned*)nullptr,
-                               (unsigned*)nullptr, d_flag);
+            if (nv && !check(hipMemcpyAsync(d_xyz, h_xyz, 3 * (size_t)nv * 4, hipMemcpyHostToDevice, s), "upload"))
+                return false;
+            if (!check(hipMemcpyAsync(d_faces, h_faces, 3 * (size_t)nf * 4, hipMemcpyHostToDevice, s), "upload"))
+                return false;
+            hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, d_nbig, (size_t)2, 0u);
+            hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nf, 256)), dim3(256), 0, s, d_cursor, (size_t)nf, 0u);
+            hipLaunchKernelGGL(classify_kernel, dim3(blocks_for(nf, 1024)), dim3(1024), 0, s, g, d_xyz, d_faces, nf,
+                               d_big, d_nbig);
+            hipLaunchKernelGGL(face_overlap_kernel, dim3(face_blocks), dim3(256), 0, s, g, d_xyz, d_faces, nf, d_masks,
+                               d_count);
+            big_overlap_kernel<false, false><<<mid_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, d_count,
+                                                                      nullptr, nullptr, nullptr, nullptr);
+            big_overlap_kernel<true, false><<<huge_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, d_count,
+                                                                      nullptr, nullptr, nullptr, nullptr);
+            scan(d_count, nf, d_first);
             hipLaunchKernelGGL(pack_faces_kernel, dim3(blocks_for(nf, 256)), dim3(256), 0, s, d_xyz, d_faces, nf,
                                reinterpret_cast<float4*>(out.tris));
+            if (!check(hipGetLastError(), "overlap launch") ||
+                !check(hipMemcpyAsync(&total, d_total, 8, hipMemcpyDeviceToHost, s), "total") ||
+                !check(hipStreamSynchronize(s), "overlap"))
+                return false;
+            if (total > 0xFFFFFFFFull) {
+                err = "grid has more than 2^32 face references; lower the resolution";
+                return false;
+            }
         }
-        hipLaunchKernelGGL(scan_local_kernel, dim3((unsigned)nb), dim3(256), 0, s, d_count, nc, d_local, d_bsum);
-        hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, s, d_bsum, nb, d_total);
-        hipLaunchKernelGGL(scan_finish_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s, d_local, d_bsum, nc,
-                           out.cell_start);
-        if (!check(hipGetLastError(), "count/scan launch")) break;
-        unsigned long long total = 0;
-        if (!check(hipMemcpyAsync(&total, d_total, 8, hipMemcpyDeviceToHost, s), "total") ||
-            !check(hipStreamSynchronize(s), "count/scan"))
-            break;
-        if (total > 0xFFFFFFFFull) {
-            err = "grid has more than 2^32 face references; lower the resolution";
-            break;
-        }
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, out.cell_start + nc, (size_t)1,
-                           (unsigned)total);
-        if (!check(hipMalloc(&out.cell_faces, std::max<size_t>(1, (size_t)total) * 4), "alloc")) break;
+        const int i_refs = R.add<Reference>((size_t)total), i_list = R.add<unsigned>((size_t)total);
+        if (!check(hipMalloc(&out.cell_faces, std::max<size_t>(1, (size_t)total) * 4), "alloc")) return false;
         out.refs = (size_t)total;
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s, d_count, nc, 0u);
-        if (nf) {
-            hipLaunchKernelGGL(grid_cells_kernel<true>, dim3(blocks_for(nf, 256)), dim3(256), 0, s, g, d_xyz,
-                               d_faces, nf, d_count, (const unsigned*)out.cell_start, out.cell_faces, d_flag, d_big,
-                               d_nbig);
-            hipLaunchKernelGGL(grid_cells_big_kernel<true>, dim3(big_blocks), dim3(256), 0, s, g, d_xyz, d_faces,
-                               (const unsigned*)d_big, (const unsigned*)d_nbig, d_count,
-                               (const unsigned*)out.cell_start, out.cell_faces, d_flag);
+        if (total) {
+            if (!check(R.allocate(), "alloc")) return false;
+            Reference* d_refs = R.get<Reference>(i_refs);
+            unsigned* d_list = R.get<unsigned>(i_list);
+            hipLaunchKernelGGL(face_place_kernel, dim3(face_blocks), dim3(256), 0, s, g, d_xyz, d_faces, nf,
+                               (const unsigned short*)d_masks, (const unsigned*)d_first, d_cells, d_refs);
+            big_overlap_kernel<false, true><<<mid_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, nullptr,
+                                                                     d_first, nullptr, d_cells, d_refs);
+            big_overlap_kernel<true, true><<<huge_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, nullptr,
+                                                                     d_first, d_cursor, d_cells, d_refs);
+            scan(d_cells, nc, out.cell_start);
+            hipLaunchKernelGGL(list_kernel, dim3(blocks_for((size_t)total, 256)), dim3(256), 0, s,
+                               (const Reference*)d_refs, (size_t)total, (const unsigned*)out.cell_start, d_list);
+            hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, out.cell_start + nc, (size_t)1,
+                               (unsigned)total);
+            hipLaunchKernelGGL(rank_kernel, dim3(blocks_for((size_t)total, 256)), dim3(256), 0, s,
+                               (const Reference*)d_refs, (size_t)total, (const unsigned*)out.cell_start,
+                               (const unsigned*)d_list, out.cell_faces);
+        } else {
+            hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc + 1, 256)), dim3(256), 0, s, out.cell_start, nc + 1,
+                               0u);
         }
-        hipLaunchKernelGGL(sort_cells_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s,
-                           (const unsigned*)out.cell_start, nc, out.cell_faces);
-        hipLaunchKernelGGL(dist_x_kernel, dim3(blocks_for(ny * nz, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(dist_x_kernel, dim3(blocks_for(ny * nz, 4)), dim3(256), 0, s,
                            (const unsigned*)out.cell_start, (int)nx, ny * nz, out.dist);
-        hipLaunchKernelGGL(dist_minmax_kernel, dim3(blocks_for(nz * nx, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(dist_minmax_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s,
                            (const unsigned char*)out.dist, d_tmp, (int)nx, (int)ny, (int)nz, 1);
-        hipLaunchKernelGGL(dist_minmax_kernel, dim3(blocks_for(ny * nx, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(dist_minmax_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s,
                            (const unsigned char*)d_tmp, out.dist, (int)nx, (int)ny, (int)nz, 2);
-        if (!check(hipGetLastError(), "fill/distance launch")) break;
-        unsigned flag = 0;
-        if (!check(hipMemcpyAsync(&flag, d_flag, 4, hipMemcpyDeviceToHost, s), "flag") ||
-            !check(hipStreamSynchronize(s), "fill/distance"))
-            break;
-        if (flag) {
-            err = "device grid build: count and fill passes disagree";
-            break;
-        }
-        ok = true;
-    } while (false);
-    for (void* p : {(void*)d_xyz, (void*)d_faces, (void*)d_count, (void*)d_local, (void*)d_bsum, (void*)d_total,
-                    (void*)d_flag, (void*)d_tmp, (void*)d_big, (void*)d_nbig})
-        if (p) (void)hipFree(p);
-    if (!ok) out.release();
+        return check(hipGetLastError(), "place/distance launch") &&
+               check(hipStreamSynchronize(s), "place/distance");
+    };
+    const bool ok = build();
+    if (!ok) {
+        (void)hipStreamSynchronize(s);  // nothing may still run on what is freed
+        out.release();
+    }
     return ok;
 }
 

@@ -67,3 +67,42 @@ def test_device_grid_renders_the_same_frame():
         assert np.array_equal(a.final, b.final)
     finally:
         view.close()
+
+
+def _lists(v, f, res=0):
+    """The grid of (v, f) from either builder, and from the automatic choice."""
+    out = []
+    with L.MainView(16, 16) as view:
+        view.set_accel(L.ACCEL_GRID, res)
+        view.update_model(v, f)
+        for b in (L.GRID_BUILD_HOST, L.GRID_BUILD_DEVICE, L.GRID_BUILD_AUTO):
+            out.append(_grid(view, b))
+    return out
+
+
+@pytest.mark.parametrize("shape", ["wall", "crowd", "slab", "wide_rows", "one"])
+def test_device_grid_edges(shape):
+    """Faces and grids at the builder's edges: one face over most cells (spread over the blocks),
+    hundreds of faces in one cell (long lists to rank), a flat mesh (one cell layer), rows longer
+    than eight 64-cell chunks with empty stretches beyond the distance's cap of 255, one face."""
+    rng = np.random.default_rng(11)
+    res = 0
+    if shape == "wall":
+        v = np.array([[-1, -1, -1], [1, 1, -0.9], [-1, 1, 1], [0.9, -1, 1]], np.float32)
+        f = np.array([[0, 1, 2], [1, 2, 3], [0, 3, 2]], np.uint32)
+    elif shape == "crowd":  # 700 small faces inside one cell of a grid that another face stretches
+        v = np.concatenate([rng.uniform(0.0, 1e-3, (2100, 3)), [[4, 4, 4], [4, 3.9, 4], [3.9, 4, 4]]]).astype(np.float32)
+        f = np.arange(2103, dtype=np.uint32).reshape(-1, 3)[rng.permutation(701)]
+    elif shape == "slab":
+        v = np.concatenate([rng.uniform(-1, 1, (300, 2)), np.zeros((300, 1))], 1).astype(np.float32)
+        f = rng.integers(0, 300, (257, 3)).astype(np.uint32)
+    elif shape == "wide_rows":
+        v = np.array([[0, 0, 0], [0.01, 0, 0], [0, 0.01, 0.01], [1, 0.02, 0.03], [0.99, 0, 0.01], [1, 0, 0]], np.float32)
+        f = np.arange(6, dtype=np.uint32).reshape(2, 3)
+        res = 700
+    else:
+        v, f = np.eye(3, dtype=np.float32), np.array([[0, 1, 2]], np.uint32)
+    print(f"[case] grid edges {shape} ({len(f)} faces)", flush=True)
+    h, d, auto = _lists(v, f, res)
+    for k in ("dims", "cell_start", "cell_faces", "dist", "tris"):
+        assert np.array_equal(h[k], d[k]) and np.array_equal(h[k], auto[k]), k
