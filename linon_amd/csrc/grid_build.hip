@@ -465,7 +465,8 @@ __global__ void __launch_bounds__(256) dist_minmax_kernel(const unsigned char* i
     const size_t s = axis == 1 ? (size_t)nx : (size_t)nx * ny;
     const unsigned char* p = in + cell;
     int best = *p;
-    for (int dlt = 1; dlt < best; ++dlt) {
+    // (past both ends of the line nothing is left that could be smaller)
+    for (int dlt = 1; dlt < best && (i - dlt >= 0 || i + dlt < n); ++dlt) {
         int g = 255;
         if (i - dlt >= 0) g = min(g, (int)p[-(ptrdiff_t)((size_t)dlt * s)]);
         if (i + dlt < n) g = min(g, (int)p[(size_t)dlt * s]);
