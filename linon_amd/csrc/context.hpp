@@ -65,8 +65,6 @@ struct Surrogate {
     float *d_col_part = nullptr, *d_out_part = nullptr;  // row sums of the bias and output-layer gradients
     // frame
     int frame_px = 0;
-    float* f_entry = nullptr;
-    int* f_entered = nullptr;
     float* f_states = nullptr;
     int* f_texel = nullptr;
     int* f_count = nullptr;

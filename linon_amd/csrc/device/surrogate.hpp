@@ -63,8 +63,9 @@ struct ApproachParams {
     StepParams step;        // escape mode, need_mapping
     float radius;
     int tiles_x;
-    float* entry_states;    // [W*H][6]: (p_entry, q) of rays that entered, by texel
-    int* entered;           // [W*H]: 1 entered, 0 finished outside the sphere
+    float* states;          // [W*H][6]: (p_entry, q) of the rays that entered, a compacted list
+    int* texel_of;          // [W*H]: the list's texels
+    int* count;             // the list's length (zeroed beforehand)
     float* mapping;         // [W*H] float4: final point of rays that never entered
     int* steps;             // [W*H] RK4 iterations spent
     int q_is_v0;            // 1: the field reads v0 (q = v0), 0: it reads v (q = current direction)
@@ -77,6 +78,12 @@ struct InsideSphere {
 
 // Integrates a camera ray until it is inside the sphere (|p| < R) or finished (escape test,
 // max_steps).  Fields act outside the sphere too, so this leg is plain RK4.
+//
+// The rays that entered are appended to one list, those of a wave's 8x8 tile together, so the RK4
+// legs that run over the list (coarse flow map, fallback, re-judging) see neighbouring pixels
+// side by side in a wave.  One atomic per wave: they all go to one address, about 9 ns each, which
+// is hidden here behind the integration (a pass of its own over a 1080p image waited 290 us for
+// them, and read and wrote 100 MB of entry states again).
 template <class F>
 __device__ void approach_body(const ApproachParams& A) {
     const int lane = threadIdx.x & 63;
@@ -105,14 +112,19 @@ __device__ void approach_body(const ApproachParams& A) {
     }
     const size_t texel = (size_t)(A.cam.height - 1 - gy) * A.cam.width + gx;
     A.steps[texel] = r.iters;
-    if (entered && !done) {
+    const bool in = entered && !done;
+    const unsigned long long lanes = __ballot(in);
+    if (in) {
+        const int first = __ffsll((long long)lanes) - 1;
+        int slot = 0;
+        if (lane == first) slot = atomicAdd(A.count, __popcll(lanes));
+        slot = __shfl(slot, first, 64) + __popcll(lanes & ((1ull << lane) - 1ull));
         const vec3 q = A.q_is_v0 ? r.v0 : r.d;
-        float* s = A.entry_states + 6 * texel;
+        float* s = A.states + 6 * (size_t)slot;
         s[0] = r.p.x; s[1] = r.p.y; s[2] = r.p.z;
         s[3] = q.x;   s[4] = q.y;   s[5] = q.z;
-        A.entered[texel] = 1;
+        A.texel_of[slot] = (int)texel;
     } else {
-        A.entered[texel] = 0;
         reinterpret_cast<float4*>(A.mapping)[texel] = make_float4(r.p.x, r.p.y, r.p.z, 1.0f);
     }
 }

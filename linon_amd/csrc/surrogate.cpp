@@ -65,7 +65,7 @@ void Surrogate::release() {
     }
     void* bufs[] = {d_wpack, d_bpack, d_freqs, d_states, d_targets, d_tscaled, d_feat, d_act[0], d_act[1], d_act[2],
                     d_act[3], d_dz[0], d_dz[1], d_dz[2], d_dz[3], d_z, d_dout, d_part, d_loss, d_col_part, d_out_part,
-                    f_entry, f_entered, f_states, f_texel, f_count, f_pred, f_accepted, f_list, f_exits, f_errs, f_feat,
+                    f_states, f_texel, f_count, f_pred, f_accepted, f_list, f_exits, f_errs, f_feat,
                     f_act0, f_act1, f_out, f_steps, f_base, f_mask};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
@@ -505,9 +505,10 @@ linon_status Context::surrogate_eval(const float* states, const float* targets, 
 }
 
 // One surrogate frame of the current view (no mesh: the mapping texture and the overlay):
-//   1. RK4 from the camera to the bounding sphere (rays that never enter end there);
-//   2. compaction of the rays that entered; the coarse flow map of their entry states (the
-//      multi-fidelity form) and the MLP, accepting confident predictions;
+//   1. RK4 from the camera to the bounding sphere (rays that never enter end there), which lists
+//      the rays that entered;
+//   2. the coarse flow map of their entry states (the multi-fidelity form) and the MLP, accepting
+//      confident predictions;
 //   3. RK4 from the entry state for rays below the confidence threshold;
 //   4. the overlay's Lyapunov exponent on that mapping; accepted rays above the threshold go
 //      to RK4 as well, and the overlay runs again;
@@ -528,8 +529,6 @@ linon_status Context::surrogate_frame(hipStream_t s) {
     const bool capturing = cap != hipStreamCaptureStatusNone;
     if (S.frame_px != npx) {
         if (capturing) return fail(LINON_ERR_STATE, "render_surrogate: render once at this size before capturing");
-        LS_CHECK(this, dalloc(S.f_entry, (size_t)npx * 6));
-        LS_CHECK(this, dalloc(S.f_entered, (size_t)npx));
         LS_CHECK(this, dalloc(S.f_states, (size_t)npx * 6));
         LS_CHECK(this, dalloc(S.f_texel, (size_t)npx));
         LS_CHECK(this, dalloc(S.f_count, 4));
@@ -569,13 +568,13 @@ linon_status Context::surrogate_frame(hipStream_t s) {
     A.step = I;
     A.radius = S.cfg.radius;
     A.tiles_x = (W + LINON_TILE - 1) / LINON_TILE;
-    A.entry_states = S.f_entry;
-    A.entered = S.f_entered;
+    A.states = S.f_states;
+    A.texel_of = S.f_texel;
+    A.count = n_in;
     A.mapping = d_mapping;
     A.steps = d_steps;
     A.q_is_v0 = q_is_v0 ? 1 : 0;
     LS_CHECK(this, wgsl ? linon_wgslmath::sg_approach(kf, A, s) : sg_approach(kf, A, s));
-    LS_CHECK(this, sg_compact_entered(S.f_entered, S.f_entry, W, H, S.f_states, S.f_texel, n_in, s));
     LS_CHECK(this, mark(1));
     // 2. coarse flow map (multi-fidelity form), then the MLP in one fused launch
     const bool coarse = S.cfg.coarse_h > 0.0f;

@@ -76,14 +76,42 @@ __global__ void __launch_bounds__(256) sample_states_kernel(unsigned long long s
     o[3] = qx; o[4] = qy; o[5] = qz;
 }
 
+// Appends to a list: every thread of the block calls it (blockDim.x = LS_LIST_BLOCK), those with
+// `want` get their slots, in thread order.  One atomic per block: all blocks' go to one address,
+// about 9 ns each, which a 1080p frame's kernels with an atomic per wave spent their time on
+// (re-judge picks 182 us).
+#define LS_LIST_BLOCK 1024
+__device__ __forceinline__ int append_slot(bool want, int* count) {
+    __shared__ int base[LS_LIST_BLOCK / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const unsigned long long lanes = __ballot(want);
+    if (lane == 0) base[wave] = __popcll(lanes);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int w = 0; w < LS_LIST_BLOCK / 64; ++w) n += base[w];
+        int at = n ? atomicAdd(count, n) : 0;
+        for (int w = 0; w < LS_LIST_BLOCK / 64; ++w) {
+            const int k = base[w];
+            base[w] = at;
+            at += k;
+        }
+    }
+    __syncthreads();
+    return base[wave] + __popcll(lanes & ((1ull << lane) - 1ull));
+}
+
 // Picks roughly one accepted ray in `stride` (hash-spread) for re-judging with RK4.
-__global__ void __launch_bounds__(256) pick_rejudge_kernel(const int* accepted, int n, const int* n_dev, int stride,
-                                                           unsigned long long seed, int* list, int* count) {
+__global__ void __launch_bounds__(LS_LIST_BLOCK) pick_rejudge_kernel(const int* accepted, int n, const int* n_dev,
+                                                                     int stride, unsigned long long seed, int* list,
+                                                                     int* count) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (n_dev ? *n_dev : n) || !accepted[i]) return;
-    if ((int)(u01(seed, (unsigned long long)i) * (float)stride) != 0) return;
-    int slot = atomicAdd(count, 1);
-    list[slot] = i;
+    const int rows = n_dev ? *n_dev : n;
+    if ((int)(blockIdx.x * blockDim.x) >= rows) return;  // the whole block
+    const bool pick =
+        i < rows && accepted[i] && (int)(u01(seed, (unsigned long long)i) * (float)stride) == 0;
+    const int slot = append_slot(pick, count);
+    if (pick) list[slot] = i;
 }
 
 // Network targets of the training set: (exit - base) * scale, per row (point scale for the
@@ -170,58 +198,31 @@ __global__ void __launch_bounds__(256) reduce_partials_kernel(const float* part,
 // Surrogate verdict per entered ray: accept (write the exit point to the mapping) when the
 // confidence reaches the threshold; otherwise queue the ray for RK4.  The exit point is the
 // base (coarse flow map, or 0) plus the output over the point scale.
-__global__ void __launch_bounds__(256) accept_kernel(const float* out, const float* base, const int* texel_of, int n,
-                                                     const int* n_dev, float scale_p, float conf_threshold,
-                                                     float* mapping, float* pred_exit, int* fallback,
-                                                     int* n_fallback, int* accepted) {
+__global__ void __launch_bounds__(LS_LIST_BLOCK) accept_kernel(const float* out, const float* base,
+                                                               const int* texel_of, int n, const int* n_dev,
+                                                               float scale_p, float conf_threshold, float* mapping,
+                                                               float* pred_exit, int* fallback, int* n_fallback,
+                                                               int* accepted) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (n_dev ? *n_dev : n)) return;
-    const float* o = out + (size_t)i * LS_OUT;
-    const float conf = 1.0f / (1.0f + __expf(-o[6]));
-    const int texel = texel_of[i];
-    const float inv = 1.0f / scale_p;
-    const float* b = base ? base + 6 * (size_t)i : nullptr;
-    const float px = (b ? b[0] : 0.0f) + o[0] * inv, py = (b ? b[1] : 0.0f) + o[1] * inv,
-                pz = (b ? b[2] : 0.0f) + o[2] * inv;
-    pred_exit[3 * (size_t)i] = px;
-    pred_exit[3 * (size_t)i + 1] = py;
-    pred_exit[3 * (size_t)i + 2] = pz;
-    if (conf >= conf_threshold) {
-        reinterpret_cast<float4*>(mapping)[texel] = make_float4(px, py, pz, 1.0f);
-        accepted[i] = 1;
-    } else {
-        accepted[i] = 0;
-        int slot = atomicAdd(n_fallback, 1);
-        fallback[slot] = i;
+    const int rows = n_dev ? *n_dev : n;
+    if ((int)(blockIdx.x * blockDim.x) >= rows) return;  // the whole block
+    bool accept = true;
+    if (i < rows) {
+        const float* o = out + (size_t)i * LS_OUT;
+        const float conf = 1.0f / (1.0f + __expf(-o[6]));
+        const float inv = 1.0f / scale_p;
+        const float* b = base ? base + 6 * (size_t)i : nullptr;
+        const float px = (b ? b[0] : 0.0f) + o[0] * inv, py = (b ? b[1] : 0.0f) + o[1] * inv,
+                    pz = (b ? b[2] : 0.0f) + o[2] * inv;
+        pred_exit[3 * (size_t)i] = px;
+        pred_exit[3 * (size_t)i + 1] = py;
+        pred_exit[3 * (size_t)i + 2] = pz;
+        accept = conf >= conf_threshold;
+        accepted[i] = accept ? 1 : 0;
+        if (accept) reinterpret_cast<float4*>(mapping)[texel_of[i]] = make_float4(px, py, pz, 1.0f);
     }
-}
-
-// Compacts the rays that entered the sphere into a prefix of entry-state rows; texel_of[i]
-// remembers where ray i's result goes.  Threads walk the image in the approach kernel's 8x8
-// tile order, one wave per tile, so each wave appends one tile's entering rays together: the
-// RK4 legs that run over the compacted rows (coarse flow map, fallback, re-judging) then see
-// neighbouring pixels side by side in a wave, as the plain kernel's tiles do, rather than 64
-// pixels of one image row.
-__global__ void __launch_bounds__(256) compact_entered_kernel(const int* entered, const float* entry_states, int W,
-                                                              int H, float* states, int* texel_of, int* count) {
-    const int lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int tiles_x = (W + LINON_TILE - 1) / LINON_TILE;
-    const int gx = (tile % tiles_x) * LINON_TILE + (lane & (LINON_TILE - 1));
-    const int gy = (tile / tiles_x) * LINON_TILE + (lane / LINON_TILE);
-    const int t = (H - 1 - gy) * W + gx;  // the approach kernel's texel of (gx, gy)
-    const bool e = gx < W && gy < H && entered[t];
-    // wave-aggregated append: one atomic per wave, lanes placed by their rank among the
-    // entering lanes of the wave
-    const unsigned long long mask = __ballot(e);
-    int base = 0;
-    if (lane == 0 && mask) base = atomicAdd(count, __popcll(mask));
-    base = __shfl(base, 0, 64);
-    if (e) {
-        const int slot = base + __popcll(mask & ((1ull << lane) - 1ull));
-        for (int k = 0; k < 6; ++k) states[6 * (size_t)slot + k] = entry_states[6 * (size_t)t + k];
-        texel_of[slot] = t;
-    }
+    const int slot = append_slot(!accept, n_fallback);
+    if (!accept) fallback[slot] = i;
 }
 
 // Rays re-judged by RK4 or sent to RK4: write the RK4 exit into the mapping; for re-judged
@@ -240,15 +241,16 @@ __global__ void __launch_bounds__(256) apply_rk4_kernel(const int* list, int n, 
 
 // Accepted rays whose Lyapunov exponent (from the surrogate's own mapping) is above the
 // threshold are queued for RK4 as well, and no longer count as accepted.
-__global__ void __launch_bounds__(256) lyapunov_gate_kernel(int* accepted, const int* texel_of, int n,
-                                                            const int* n_dev, const float* lyap, float threshold,
-                                                            int* list, int* count) {
+__global__ void __launch_bounds__(LS_LIST_BLOCK) lyapunov_gate_kernel(int* accepted, const int* texel_of, int n,
+                                                                      const int* n_dev, const float* lyap,
+                                                                      float threshold, int* list, int* count) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (n_dev ? *n_dev : n) || !accepted[i]) return;
-    const float l = lyap[texel_of[i]];
-    if (l > threshold) {
+    const int rows = n_dev ? *n_dev : n;
+    if ((int)(blockIdx.x * blockDim.x) >= rows) return;  // the whole block
+    const bool gate = i < rows && accepted[i] && lyap[texel_of[i]] > threshold;
+    const int slot = append_slot(gate, count);
+    if (gate) {
         accepted[i] = 0;
-        int slot = atomicAdd(count, 1);
         list[slot] = i;
     }
 }
@@ -284,6 +286,7 @@ hipError_t sg_gemm(const lm::GemmParams& P, int splits, hipStream_t s) {
 }
 
 #define LS_GRID(n) dim3(((n) + 255) / 256), dim3(256)
+#define LS_LIST_GRID(n) dim3(((n) + LS_LIST_BLOCK - 1) / LS_LIST_BLOCK), dim3(LS_LIST_BLOCK)
 
 hipError_t sg_mlp_pack(const float* W, int K, u16* dst, bool transposed, hipStream_t s) {
     if (transposed)
@@ -342,15 +345,8 @@ hipError_t sg_update(const lm::UpdateParams& P, hipStream_t s) {
 hipError_t sg_accept(const float* out, const float* base, const int* texel_of, int n, const int* n_dev, float scale_p,
                      float thr, float* mapping, float* pred_exit, int* fallback, int* n_fallback, int* accepted,
                      hipStream_t s) {
-    hipLaunchKernelGGL(accept_kernel, LS_GRID(n), 0, s, out, base, texel_of, n, n_dev, scale_p, thr, mapping,
+    hipLaunchKernelGGL(accept_kernel, LS_LIST_GRID(n), 0, s, out, base, texel_of, n, n_dev, scale_p, thr, mapping,
                        pred_exit, fallback, n_fallback, accepted);
-    return hipGetLastError();
-}
-hipError_t sg_compact_entered(const int* entered, const float* entry_states, int W, int H, float* states,
-                              int* texel_of, int* count, hipStream_t s) {
-    const unsigned tiles = (unsigned)(((W + LINON_TILE - 1) / LINON_TILE) * ((H + LINON_TILE - 1) / LINON_TILE));
-    hipLaunchKernelGGL(compact_entered_kernel, dim3((tiles + 3) / 4), dim3(256), 0, s, entered, entry_states, W, H,
-                       states, texel_of, count);
     return hipGetLastError();
 }
 hipError_t sg_apply_rk4(const int* list, int n, const int* n_dev, const float* exits, const int* texel_of,
@@ -367,7 +363,7 @@ hipError_t sg_accepted_mask(const int* accepted, const int* texel_of, int n, con
 }
 hipError_t sg_lyapunov_gate(int* accepted, const int* texel_of, int n, const int* n_dev, const float* lyap, float thr,
                             int* list, int* count, hipStream_t s) {
-    hipLaunchKernelGGL(lyapunov_gate_kernel, LS_GRID(n), 0, s, accepted, texel_of, n, n_dev, lyap, thr, list, count);
+    hipLaunchKernelGGL(lyapunov_gate_kernel, LS_LIST_GRID(n), 0, s, accepted, texel_of, n, n_dev, lyap, thr, list, count);
     return hipGetLastError();
 }
 hipError_t sg_sample_states(unsigned long long seed, int n, float radius, float inset, float* states, hipStream_t s) {
@@ -376,7 +372,7 @@ hipError_t sg_sample_states(unsigned long long seed, int n, float radius, float 
 }
 hipError_t sg_pick_rejudge(const int* accepted, int n, const int* n_dev, int stride, unsigned long long seed, int* list,
                            int* count, hipStream_t s) {
-    hipLaunchKernelGGL(pick_rejudge_kernel, LS_GRID(n), 0, s, accepted, n, n_dev, stride, seed, list, count);
+    hipLaunchKernelGGL(pick_rejudge_kernel, LS_LIST_GRID(n), 0, s, accepted, n, n_dev, stride, seed, list, count);
     return hipGetLastError();
 }
 hipError_t sg_fill_i32(int* p, int n, int value, hipStream_t s) {
