@@ -394,13 +394,7 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     auto quot = [](float a, float b) { return InRange ? div_in_range(a, b) : a / b; };
     float eta_in = quot(refraction_index_num(t_in), refraction_index_den(t_in));
     float eta_out = quot(refraction_index_num(t_out), refraction_index_den(t_out));
-    float cosi = clamp(-1.0f, 1.0f, dot(v_in, n));
-    vec3 n_ref = n;
-    if (cosi < 0.0f) {
-        cosi = -cosi;
-    } else {
-        n_ref = -n;
-    }
+    const float cosi = clamp(-1.0f, 1.0f, dot(v_in, n));
     float eta = quot(eta_in, eta_out);
     // k = RN(1 - e t), e = RN(eta eta), t = RN(1 - cosi cosi) in [0, 1] (the FMA form the
     // contracted expression 1 - eta * eta * (1 - cosi * cosi) compiles to).  k is never in
@@ -408,17 +402,25 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     // exponents of e and t add up to at least -2 and e t is a multiple of 2^-48, as is 1 - e t.
     // The root therefore needs no rescaling of tiny operands.
     const float k = __builtin_fmaf(-(eta * eta), __builtin_fmaf(-cosi, cosi, 1.0f), 1.0f);
-    // eta v_in + (eta cosi - sqrt(k)) n_ref with its contraction written out, fma(eta, v_i,
-    // RN(X n_i)), X = fma(eta, cosi, -sqrt(k)): the form the compiler picks for the expression, so
-    // that it no longer depends on that pick.  NaN where k < 0.
-    const float X = __builtin_fmaf(eta, cosi, -sqrt_rn_no_tiny(k));
-    vec3 out = {__builtin_fmaf(eta, v_in.x, mul_rounded(X, n_ref.x)),
-                __builtin_fmaf(eta, v_in.y, mul_rounded(X, n_ref.y)),
-                __builtin_fmaf(eta, v_in.z, mul_rounded(X, n_ref.z))};
+    // The shader's eta v_in + (eta |cosi| - sqrt(k)) n_ref, n_ref = n where cosi < 0 and -n
+    // elsewhere, with its contraction written out: fma(eta, v_i, RN(X n_ref_i)), X = fma(eta, |cosi|,
+    // -sqrt(k)) (the form the compiler picked for the expression).  Rounding is symmetric in sign,
+    // so X and n_ref may both change sign together: X n_ref = Y n with Y = fma(-eta, cosi, +-sqrt(k)),
+    // the root negated where cosi < 0.  One select instead of a branch over the side: its exec mask
+    // and moves took about 25 cycles a stage where a wave has its SIMD to itself (96x64 hot air's
+    // sample rays 5.3 -> 4.9 ms; 1080p hot air 13.55 -> 13.47 ms, plane mirage 13.55 -> 12.48).  With
+    // copysign(root, cosi) in place of the select, 1080p hot air takes 13.85.  NaN where k < 0.
+    const float root = sqrt_rn_no_tiny(k);
+    const float Y = __builtin_fmaf(-eta, cosi, cosi < 0.0f ? -root : root);
+    vec3 out = {__builtin_fmaf(eta, v_in.x, mul_rounded(Y, n.x)),
+                __builtin_fmaf(eta, v_in.y, mul_rounded(Y, n.y)),
+                __builtin_fmaf(eta, v_in.z, mul_rounded(Y, n.z))};
     // total internal reflection (k < 0) on any lane: a wave-uniform branch, so that waves
     // without it (nearly all) carry no reflection code, not even with an empty lane mask
+    // (the empty asm keeps the compiler from turning the branch into selects)
     if (__any(k < 0.0f)) {
-        const vec3 r = reflect(v_in, n_ref);
+        asm volatile("");
+        const vec3 r = reflect(v_in, n);  // = reflect(v_in, -n)
         const bool tir = k < 0.0f;
         out = {tir ? r.x : out.x, tir ? r.y : out.y, tir ? r.z : out.z};
     }
@@ -436,8 +438,8 @@ __device__ __forceinline__ vec3 refraction_in_range(float t_in, float t_out, vec
 // of a field that compares T(p_prev) with T(p).  The index ratio n(t) / n(t) is then exactly 1
 // (a correctly rounded x / x), so its quotients and every product with it drop out:
 //   k = fma(-(eta eta), fma(-cosi, cosi, 1), 1)  ->  1 - fma(-cosi, cosi, 1)
-//   X = fma(eta, cosi, -sqrt(k))                 ->  cosi - sqrt(k)
-//   fma(v_in, eta, RN(X n))                      ->  v_in + RN(X n)
+//   Y = fma(-eta, cosi, +-sqrt(k))               ->  +-sqrt(k) - cosi
+//   fma(v_in, eta, RN(Y n))                      ->  v_in + RN(Y n)
 // which is how refraction_impl's expression compiles, so the result is the same bit for bit.  A
 // NaN t gives NaN in every component, as its NaN ratio does there (cosi - (t - t) is cosi for
 // a finite t).  The WGSL-accuracy build divides approximately, where n(t) / n(t) need not be
@@ -446,23 +448,19 @@ __device__ __forceinline__ vec3 refraction_in_range_same(float t, vec3 v_in, vec
 #ifdef LINON_FAST_MATH
     return refraction_impl<true>(t, t, v_in, n);
 #else
-    float cosi = clamp(-1.0f, 1.0f, dot(v_in, n)) - (t - t);
-    vec3 n_ref = n;
-    if (cosi < 0.0f) {
-        cosi = -cosi;
-    } else {
-        n_ref = -n;
-    }
+    const float cosi = clamp(-1.0f, 1.0f, dot(v_in, n)) - (t - t);
     // 1 - t with t = RN(1 - cosi cosi) in [0, 1]: zero, or at least 2^-24 (t >= 1/2 is a
     // multiple of 2^-24) -- no tiny operand for the root; never negative, so never the total
     // internal reflection of the general form (a NaN t gives NaN there as here)
     const float k = 1.0f - __builtin_fmaf(-cosi, cosi, 1.0f);
-    const float x = cosi - sqrt_rn_no_tiny(k);
+    // (the sign here by copysign, of cosi + 0 since -0 is not < 0: 1080p hot air takes 13.9 ms with a
+    // select in this stage too, 13.5 with it in the general form alone)
+    const float y = __builtin_copysignf(sqrt_rn_no_tiny(k), cosi + 0.0f) - cosi;
     auto axpy = [](float a, float b, float c) {
 #pragma clang fp contract(off)
         return a * b + c;
     };
-    return {axpy(x, n_ref.x, v_in.x), axpy(x, n_ref.y, v_in.y), axpy(x, n_ref.z, v_in.z)};
+    return {axpy(y, n.x, v_in.x), axpy(y, n.y, v_in.y), axpy(y, n.z, v_in.z)};
 #endif
 }
 __device__ __forceinline__ float point_plane_distance(vec3 p, vec3 n, vec3 p0) {
