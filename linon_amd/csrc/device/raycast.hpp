@@ -336,11 +336,46 @@ __device__ __forceinline__ vec3 rk4_stage1(const F& f, vec3 p, vec3 v0, vec3 v, 
     return f(p, p, v0, v, t);
 }
 
+struct Rgb {
+    float r, g, b;
+};
+
+// Steps of one sample ray from p along d: the position before every stride-th step recorded, nsamp
+// of them.  One wave runs this for thousands of dependent steps, so its length in instructions is
+// a small frame's time: the records are counted down rather than found by dividing the step index
+// (about 30 instructions a step; swirl's 5000 steps 1.26 -> 0.95 ms, hot air's 4.0 -> 3.5), and
+// nothing is integrated past the last one.  One loop for every field weight: a second one for
+// weight 1 saves six instructions a step here but slows the pixels' loop of the same kernel by
+// 2.5% (1080p hot air 13.6 -> 13.95 ms).
+template <class F>
+__device__ __forceinline__ void sample_ray_steps(vec3 p, vec3 d, float w, int nsamp, int stride, float4* out,
+                                                 Rgb colour) {
+    const F field{};
+    const vec3 start_dir = d;
+    const float h = 0.001f, hh = rn::mul(0.5f, h);
+    float t = 0.0f;
+    for (int left = nsamp;;) {
+        out[0] = make_float4(p.x, p.y, p.z, 1.0f);
+        out[1] = make_float4(colour.r, colour.g, colour.b, 0.5f);
+        if (--left <= 0) return;
+        out += 2;
+        for (int i = 0; i < stride; ++i) {
+            vec3 k1 = rk4_stage1(field, p, start_dir, d, t, 0);
+            vec3 k2 = field(p, rn::add(p, rn::mul(hh, k1)), start_dir, k1, rn::add(t, hh));
+            vec3 k3 = field(p, rn::add(p, rn::mul(hh, k2)), start_dir, k2, rn::add(t, hh));
+            vec3 k4 = field(p, rn::add(p, rn::mul(h, k3)), start_dir, k3, rn::add(t, h));
+            vec3 V = rk4_average(k1, k2, k3, k4);
+            d = rn::add(rn::mul(rn::sub(1.0f, w), d), rn::mul(w, V));
+            p = rn::add(p, rn::mul(d, h));
+            t = rn::add(t, h);
+        }
+    }
+}
+
 // The 8 sample rays (src/main_view.wgsl:281-335,470-479): fixed h = 0.001, no scene queries,
 // the position before every stride-th step recorded as {(p, 1), (colour, 0.5)}.
 template <class F>
 __device__ void sample_rays(const RaycastParams& P, const CameraFrame& cam, int r) {
-    const F field{};
     float ox, oy, cr, cg, cb;
     switch (r) {
         case 0: ox = -1; oy = -1; cr = 1.0f; cg = 0.0f; cb = 0.0f; break;
@@ -367,29 +402,11 @@ __device__ void sample_rays(const RaycastParams& P, const CameraFrame& cam, int 
     float v2 = rn::sub(rn::mul(py, cam.vh), rn::mul(0.5f, cam.vh));
     vec3 s2 = rn::add(rn::add(rn::mul(u2, cam.nh), rn::mul(v2, cam.nv)), rn::mul(0.035f, cam.vd));
     const vec3 start_dir = rn::normalize(s2);
-    vec3 p = cam.origin, d = start_dir;
-    const float w = P.step.field_weight;
-    const float h = 0.001f, hh = rn::mul(0.5f, h);
-    float t = 0.0f;
     const int nsamp = P.samples_per_ray;
     const int stride = P.sample_steps / nsamp;
-    float4* out = reinterpret_cast<float4*>(P.ray_samples);
-    for (int i = 0; i < P.sample_steps; ++i) {
-        vec3 k1 = rk4_stage1(field, p, start_dir, d, t, 0);
-        vec3 k2 = field(p, rn::add(p, rn::mul(hh, k1)), start_dir, k1, rn::add(t, hh));
-        vec3 k3 = field(p, rn::add(p, rn::mul(hh, k2)), start_dir, k2, rn::add(t, hh));
-        vec3 k4 = field(p, rn::add(p, rn::mul(h, k3)), start_dir, k3, rn::add(t, h));
-        vec3 V = rk4_average(k1, k2, k3, k4);
-        d = rn::add(rn::mul(rn::sub(1.0f, w), d), rn::mul(w, V));
-        vec3 step = rn::mul(d, h);
-        if (i % stride == 0 && i / stride < nsamp) {
-            int idx = r * nsamp + i / stride;
-            out[2 * idx] = make_float4(p.x, p.y, p.z, 1.0f);
-            out[2 * idx + 1] = make_float4(cr, cg, cb, 0.5f);
-        }
-        p = rn::add(p, step);
-        t = rn::add(t, h);
-    }
+    float4* out = reinterpret_cast<float4*>(P.ray_samples) + 2 * r * nsamp;
+    const Rgb colour{cr, cg, cb};
+    sample_ray_steps<F>(cam.origin, start_dir, P.step.field_weight, nsamp, stride, out, colour);
 }
 
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
@@ -661,6 +678,8 @@ __device__ __forceinline__ void raycast_body(const RaycastParams& P) {
     const int lane = threadIdx.x;
     if (P.sample_block) {
         if (b == 0) {
+            // one wave for the 8 rays: with a block each, hence an XCD each, the slowest of the 8
+            // took 10-15% longer than the one
             if (lane < 8 && P.ray_samples && P.samples_per_ray > 0) sample_rays<F>(P, cam, lane);
             return;
         }

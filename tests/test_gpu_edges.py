@@ -117,3 +117,23 @@ def test_sample_count_not_dividing_steps(view):
     np.testing.assert_array_equal(got[:, :, 1], ref[:, :, 1])
     err = np.abs(got[:, :, 0, :3] - ref[:, :, 0, :3]) / np.maximum(1.0, np.abs(ref[:, :, 0, :3]))
     assert err.max() <= 1e-3, err.max()
+
+
+@pytest.mark.parametrize("records, steps", [(1, 1), (1, 500), (3, 3), (7, 20), (499, 500)])
+def test_sample_counts_at_the_edges(view, records, steps):
+    """One record, a record every step and strides that leave steps after the last record: record k
+    is the position before step k * (steps // records), as in one long run with a record a step."""
+    view.resize_texture(16, 16)
+    view.update_camera(L.Camera.arcball_default(scenes.reference_startup_scene()[2]))
+    view.update_settings(L.Settings.make(mouse_pos=(0.45, 0.5)))
+    view.set_field("mirage_spherical_sigmoid")
+    view.set_integrator(L.Integrator.make(samples_per_ray=500, sample_steps=500))
+    print("[case] 500 sample records", flush=True)
+    view.render()
+    every = view.read_ray_samples()
+    view.set_integrator(L.Integrator.make(samples_per_ray=records, sample_steps=steps))
+    print(f"[case] {records} sample records over {steps} steps", flush=True)
+    view.render()
+    got = view.read_ray_samples()
+    assert got.shape == (8, records, 2, 4)
+    np.testing.assert_array_equal(got, every[:, :: steps // records][:, :records])
