@@ -24,7 +24,7 @@ DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-result",
           f"-I{ROOT / 'include'}", f"-I{CSRC}"]
 
-SOURCES = ["kernels.hip", "surrogate.hip", "grid_build.hip", "noalloc.hip", "context.cpp", "grid.cpp", "jit.cpp", "wgsl.cpp", "batch.cpp", "surrogate.cpp"]
+SOURCES = ["kernels.hip", "surrogate.hip", "grid_build.hip", "noalloc.hip", "context.cpp", "grid.cpp", "jit.cpp", "wgsl.cpp", "batch.cpp", "readback.cpp", "surrogate.cpp"]
 # The ray-cast and surrogate kernels are compiled a second time with the accuracy WGSL itself
 # specifies (approximate division and sqrt, hardware transcendentals) into namespace
 # linon_wgslmath; linon_set_math chooses between the two builds per field.

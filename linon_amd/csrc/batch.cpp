@@ -198,6 +198,7 @@ linon_status Context::batch_capture() {
 }  // namespace linon
 
 using linon::Context;
+using linon::HostCopy;
 
 extern "C" {
 
@@ -243,13 +244,19 @@ linon_status linon_read_batch_view(linon_context* ctx, int view, uint8_t* rgba, 
         return c->fail(LINON_ERR_ARGUMENT, "read_batch_view: view index out of range");
     const size_t off = c->batch.view_px[view];
     const size_t n = c->batch.view_px[view + 1] - off;
-    linon_status st = LINON_OK;
-    if (rgba) st = c->read(c->batch.d_color + off, rgba, n * 4, rgba_bytes, "read_batch_view rgba");
-    if (st == LINON_OK && mapping)
-        st = c->read(c->batch.d_mapping + 4 * off, mapping, n * 16, mapping_bytes, "read_batch_view mapping");
-    if (st == LINON_OK && hit_faces)
-        st = c->read(c->batch.d_hit + off, hit_faces, n * 4, hit_bytes, "read_batch_view hit_faces");
-    if (st == LINON_OK && steps) st = c->read(c->batch.d_steps + off, steps, n * 4, steps_bytes, "read_batch_view steps");
+    HostCopy copies[4];
+    int num = 0;
+    auto add = [&](const void* src, void* dst, size_t want, size_t bytes, const char* what) {
+        if (!dst) return LINON_OK;
+        const linon_status st = c->readable(src, dst, want, bytes, what);
+        if (st == LINON_OK) copies[num++] = HostCopy{dst, src, want};
+        return st;
+    };
+    linon_status st = add(c->batch.d_color + off, rgba, n * 4, rgba_bytes, "read_batch_view rgba");
+    if (st == LINON_OK) st = add(c->batch.d_mapping + 4 * off, mapping, n * 16, mapping_bytes, "read_batch_view mapping");
+    if (st == LINON_OK) st = add(c->batch.d_hit + off, hit_faces, n * 4, hit_bytes, "read_batch_view hit_faces");
+    if (st == LINON_OK) st = add(c->batch.d_steps + off, steps, n * 4, steps_bytes, "read_batch_view steps");
+    if (st == LINON_OK) st = c->read_all(copies, num);
     return st;
 }
 

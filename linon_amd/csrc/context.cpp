@@ -264,16 +264,27 @@ bool wgsl_math_default(int math, int field) {
     }
 }
 
-linon_status Context::read(const void* src, void* dst, size_t want, size_t bytes, const char* what) {
+linon_status Context::readable(const void* src, const void* dst, size_t want, size_t bytes, const char* what) {
     if (!dst) return fail(LINON_ERR_ARGUMENT, std::string(what) + ": null destination");
     if (!src) return fail(LINON_ERR_STATE, std::string(what) + ": no buffer (the last linon_resize failed)");
     if (bytes < want)
         return fail(LINON_ERR_ARGUMENT, std::string(what) + ": buffer too small (" + std::to_string(bytes) +
                                             " < " + std::to_string(want) + ")");
+    return LINON_OK;
+}
+
+linon_status Context::read(const void* src, void* dst, size_t want, size_t bytes, const char* what) {
+    const linon_status st = readable(src, dst, want, bytes, what);
+    if (st != LINON_OK) return st;
+    const HostCopy one{dst, src, want};
+    return read_all(&one, 1);
+}
+
+linon_status Context::read_all(const HostCopy* copies, int n) {
     LN_CHECK_HIP(this, hipSetDevice(device));
     // renders may run on a caller's stream: wait for the whole device
     LN_CHECK_HIP(this, hipDeviceSynchronize());
-    LN_CHECK_HIP(this, hipMemcpy(dst, src, want, hipMemcpyDeviceToHost));
+    LN_CHECK_HIP(this, staging.copy(copies, n, stream, device));
     return LINON_OK;
 }
 
@@ -427,6 +438,7 @@ void linon_destroy(linon_context* ctx) {
     if (c->batch_fork) (void)hipEventDestroy(c->batch_fork);
     for (auto& s : c->batch_side)
         if (s) (void)hipStreamDestroy(s);
+    c->staging.release();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }

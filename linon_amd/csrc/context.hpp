@@ -7,6 +7,7 @@
 
 #include "../../include/linon.h"
 #include "device/params.hpp"
+#include "readback.hpp"
 
 namespace linon {
 
@@ -187,7 +188,10 @@ struct Context {
     void fill_raycast_params(RaycastParams& P, const linon_integrator& ig) const;
     linon_status render_with(const linon_integrator& ig, hipStream_t s);
     hipEvent_t* next_timing_slot();
+    linon_status readable(const void* src, const void* dst, size_t want, size_t bytes, const char* what);
     linon_status read(const void* src, void* dst, size_t want, size_t bytes, const char* what);
+    linon_status read_all(const HostCopy* copies, int n);
+    ReadStaging staging;
 };
 
 void fill_step(StepParams& I, const linon_integrator& ig, float field_weight);
