@@ -14,7 +14,9 @@
 //     bytes a lane, 1 KB a wave), not as a row-major matrix.
 // What bounds it: at 65536 rows, 290 MB of bf16 rows and 400 MB of z to and from memory, and the
 // SiLU and its derivative (an exponential and a reciprocal each, quarter rate) beside the MFMAs.
-// 196 us there; the launches it replaces took 895 (600 of them the dX products on 2-byte loads).
+// 189 us there; the launches it replaces took 895 (600 of them the dX products on 2-byte loads).
+// The weights of a layer are first read at its start: read under the layer before, as inference
+// does, they cost 190 bytes of spills more and the pass takes 217 us.
 //
 // The arithmetic is that of the kernels it replaces (features_body, gemm_body's k order,
 // out_layer_kernel's and loss_kernel's expressions): the same bits.
@@ -75,15 +77,14 @@ __device__ __forceinline__ void tile_out(const u16 (*tile)[LM_FUSED_LDA], int ro
 
 __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     __shared__ __attribute__((aligned(16))) u16 tile[LM_FUSED_ROWS][LM_FUSED_LDA];
-    __shared__ __attribute__((aligned(16))) float w5[LS_HIDDEN][8];     // the 7 outputs and a zero
+    __shared__ __attribute__((aligned(16))) float w5[8][LM_FUSED_W5];   // the 7 outputs and a zero
     __shared__ __attribute__((aligned(16))) float d5[LM_FUSED_ROWS][8]; // dOut of each row and a zero
     __shared__ float wave_loss[4];
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int row0 = blockIdx.x * LM_FUSED_ROWS;
     const int n = P.rows;
-    for (int i = tid; i < LS_HIDDEN * 8; i += 256)
-        w5[i >> 3][i & 7] = (i & 7) < LS_OUT ? P.w_out[(i >> 3) * LS_OUT + (i & 7)] : 0.0f;
+    mlp_stage_output(P.w_out, P.b_out, w5, tid);
 
     // ---- gather and features: two threads per row, eight frequencies each ----
     const int r = tid >> 1, half = tid & 1;
@@ -96,38 +97,11 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
         h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
         h ^= h >> 31;
         src = (size_t)(h % (unsigned long long)P.n_data);
-        float x[LS_IN];
-        const float inv_r = 1.0f / P.radius;
-        for (int k = 0; k < 3; ++k) x[k] = P.states[6 * src + k] * inv_r;
-        for (int k = 3; k < 6; ++k) x[k] = P.states[6 * src + k];
-        u16* o = tile[r];
-        if (half == 0)
-            for (int k = 0; k < LS_IN; ++k) o[k] = f2bf(x[k]);
-        for (int f = 8 * half; f < 8 * half + 8; ++f) {
-            const float w = P.freqs[f];
-            for (int k = 0; k < LS_IN; ++k) {
-                float s, c;
-                __sincosf(w * x[k], &s, &c);
-                o[LS_IN + 2 * (f * LS_IN + k)] = f2bf(s);
-                o[LS_IN + 2 * (f * LS_IN + k) + 1] = f2bf(c);
-            }
-        }
-        if (half == 1)
-            for (int k = LS_FEATS; k < LS_FEATS_PAD; ++k) o[k] = 0;
-    } else {
-        for (int k = half; k < LS_FEATS_PAD; k += 2) tile[r][k] = 0;
     }
+    mlp_features(in ? P.states + 6 * src : nullptr, P.radius, P.freqs, half, tile[r]);
     __syncthreads();
 
     f32x16 acc[2][4];
-    auto clear = [&]() {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.0f;
-    };
     // this thread's z scratch of layer l: 32 float4, 256 threads apart
     const size_t tiles = gridDim.x;
     auto zat = [&](int l) {
@@ -138,13 +112,15 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     // ---- forward ----
 #pragma nounroll
     for (int l = 0; l < 4; ++l) {
-        clear();
+        u32x4v wa[2][2], wb[2][2];
+        const u16* wl = P.wpack + pack_offset(l);
+        mlp_load_pair(wl, 0, wave, lane, wa);
         if (l == 0) {
             tile_out<LS_FEATS_PAD / 8>(tile, row0, n, P.feat);
-            mlp_layer_k<LM_FUSED_KSTEPS0>(P.wpack, tile, wave, lane, acc);
+            mlp_layer_k<LM_FUSED_KSTEPS0, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
         } else {
             tile_out<LS_HIDDEN / 8>(tile, row0, n, P.act[l - 1]);
-            mlp_layer_k<LM_FUSED_KSTEPS>(P.wpack + pack_offset(l), tile, wave, lane, acc);
+            mlp_layer_k<LM_FUSED_KSTEPS, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
         }
         __syncthreads();  // every wave has read this layer's input
         const float* bias = P.bias[l];
@@ -176,23 +152,12 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     tile_out<LS_HIDDEN / 8>(tile, row0, n, P.act[3]);
     float loss = 0.0f;
     {
+        const int ray = 64 * (wave & 1) + lane, oq = 4 * (wave >> 1);
+        *reinterpret_cast<f32x4v*>(&d5[ray][oq]) = mlp_output(tile[ray], w5, oq, lane);
+        __syncthreads();
         const int o0 = 4 * half;
-        float s[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = P.b_out[min(o0 + q, LS_OUT - 1)];
-        for (int k8 = 0; k8 < LS_HIDDEN; k8 += 8) {
-            const uint4 a8 = *reinterpret_cast<const uint4*>(&tile[r][k8]);
-            const unsigned aw[4] = {a8.x, a8.y, a8.z, a8.w};
-#pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                const float a = __uint_as_float(kk & 1 ? (aw[kk >> 1] & 0xffff0000u) : (aw[kk >> 1] << 16));
-                const float4 w = *reinterpret_cast<const float4*>(&w5[k8 + kk][o0]);
-                s[0] = __builtin_fmaf(a, w.x, s[0]);
-                s[1] = __builtin_fmaf(a, w.y, s[1]);
-                s[2] = __builtin_fmaf(a, w.z, s[2]);
-                s[3] = __builtin_fmaf(a, w.w, s[3]);
-            }
-        }
+        const float4 sv = *reinterpret_cast<const float4*>(&d5[r][o0]);
+        const float s[4] = {sv.x, sv.y, sv.z, sv.w};
         float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if (in) {
             const float* y = P.targets + 6 * src;
@@ -239,20 +204,22 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int n0 = nl + 32 * j + 8 * g;
+                float4 w[LS_OUT];
+#pragma unroll
+                for (int o = 0; o < LS_OUT; ++o) w[o] = *reinterpret_cast<const float4*>(&w5[o][n0]);
                 float t[4][4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    const float4 wa = *reinterpret_cast<const float4*>(&w5[n0 + c][0]);
-                    const float4 wb = *reinterpret_cast<const float4*>(&w5[n0 + c][4]);
+                    auto wc = [&](int o) { return c == 0 ? w[o].x : c == 1 ? w[o].y : c == 2 ? w[o].z : w[o].w; };
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float s = __builtin_fmaf(da[i].x, wa.x, 0.0f);
-                        s = __builtin_fmaf(da[i].y, wa.y, s);
-                        s = __builtin_fmaf(da[i].z, wa.z, s);
-                        s = __builtin_fmaf(da[i].w, wa.w, s);
-                        s = __builtin_fmaf(db[i].x, wb.x, s);
-                        s = __builtin_fmaf(db[i].y, wb.y, s);
-                        s = __builtin_fmaf(db[i].z, wb.z, s);
+                        float s = __builtin_fmaf(da[i].x, wc(0), 0.0f);
+                        s = __builtin_fmaf(da[i].y, wc(1), s);
+                        s = __builtin_fmaf(da[i].z, wc(2), s);
+                        s = __builtin_fmaf(da[i].w, wc(3), s);
+                        s = __builtin_fmaf(db[i].x, wc(4), s);
+                        s = __builtin_fmaf(db[i].y, wc(5), s);
+                        s = __builtin_fmaf(db[i].z, wc(6), s);
                         t[i][c] = s * silu_grad(acc[j][i][4 * g + c]);
                     }
                 }
@@ -267,9 +234,11 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     // ---- dZ of layer l - 1 = (dZ W^T) * silu'(z_{l-1}) ----
 #pragma nounroll
     for (int l = 3; l > 0; --l) {
-        clear();
+        u32x4v wa[2][2], wb[2][2];
+        const u16* wl = P.bpack + (size_t)(l - 1) * LM_PACK_LAYER;
+        mlp_load_pair(wl, 0, wave, lane, wa);
         tile_out<LS_HIDDEN / 8>(tile, row0, n, P.dz[l]);
-        mlp_layer_k<LM_FUSED_KSTEPS>(P.bpack + (size_t)(l - 1) * LM_PACK_LAYER, tile, wave, lane, acc);
+        mlp_layer_k<LM_FUSED_KSTEPS, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
         __syncthreads();
         const float4* z = zat(l - 1);
 #pragma unroll
