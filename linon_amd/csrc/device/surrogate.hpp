@@ -60,7 +60,7 @@ __device__ __forceinline__ void features_body(const SurrogateIO& S) {
 // ---- RK4 legs of a surrogate frame ------------------------------------------------------
 struct ApproachParams {
     CameraParams cam;
-    StepParams step;        // escape mode, need_mapping
+    StepParams step;        // escape mode, fixed step, field weight 1
     float radius;
     int tiles_x;
     float* states;          // [W*H][6]: (p_entry, q) of the rays that entered, a compacted list
@@ -72,8 +72,9 @@ struct ApproachParams {
 };
 
 struct InsideSphere {
+    static constexpr bool EACH_STEP = true;
     float r2;
-    __device__ __forceinline__ bool operator()(const lk::RayState& r) const { return lk::rn::dot(r.p, r.p) < r2; }
+    __device__ __forceinline__ bool operator()(const vec3& p) const { return lk::rn::dot(p, p) < r2; }
 };
 
 // Integrates a camera ray until it is inside the sphere (|p| < R) or finished (escape test,
@@ -96,18 +97,12 @@ __device__ void approach_body(const ApproachParams& A) {
     const lk::CameraFrame cam = lk::camera_frame(A.cam);
     lk::RayState r;
     lk::ray_begin(r, cam.origin, lk::camera_dir(cam, A.cam, gx, gy), A.step);
-    SceneParams none;
-    none.accel = LINON_ACCEL_BRUTE_K;
-    none.num_faces = 0;
-    none.tris = nullptr;
-    none.skip_margin = 0.0f;
     const float r2 = A.radius * A.radius;
     bool entered = lk::rn::dot(r.p, r.p) < r2;
     bool done = false;
-    lk::QueryStats st{0ull, 0u, 0u, 0u};  // no mesh: nothing is counted
     if (!entered) {
         // steps until the ray is inside the sphere (the loop's own stop test) or finished
-        done = lk::ray_advance<F>(r, A.step, none, nullptr, 0x7fffffff, st, InsideSphere{r2});
+        done = lk::ray_advance_free<F, true>(r, A.step, InsideSphere{r2});
         entered = lk::rn::dot(r.p, r.p) < r2;
     }
     const size_t texel = (size_t)(A.cam.height - 1 - gy) * A.cam.width + gx;
@@ -155,13 +150,19 @@ __device__ void flowmap_body(const FlowmapParams& P) {
     lk::ray_begin(r, vec3f(s[0], s[1], s[2]), vec3f(s[3], s[4], s[5]), P.step);
     const int before = P.iters_at ? P.iters_at[P.texel_of[slot]] : 0;
     r.iters = before;
-    SceneParams none;
-    none.accel = LINON_ACCEL_BRUTE_K;
-    none.num_faces = 0;
-    none.tris = nullptr;
-    none.skip_margin = 0.0f;
-    lk::QueryStats st{0ull, 0u, 0u, 0u};  // no mesh: nothing is counted
-    lk::ray_advance<F>(r, P.step, none, nullptr, 0x7fffffff, st);
+    if (P.step.adaptive) {  // a caller's integrator
+        SceneParams none;
+        none.accel = LINON_ACCEL_BRUTE_K;
+        none.num_faces = 0;
+        none.tris = nullptr;
+        none.skip_margin = 0.0f;
+        lk::QueryStats st{0ull, 0u, 0u, 0u};  // no mesh: nothing is counted
+        lk::ray_advance<F>(r, P.step, none, nullptr, 0x7fffffff, st);
+    } else if (P.step.field_weight == 1.0f) {
+        lk::ray_advance_free<F, true>(r, P.step);
+    } else {
+        lk::ray_advance_free<F, false>(r, P.step);
+    }
     float* o = P.exits + 6 * (size_t)slot;
     o[0] = r.p.x; o[1] = r.p.y; o[2] = r.p.z;
     o[3] = r.d.x; o[4] = r.d.y; o[5] = r.d.z;
