@@ -10,7 +10,7 @@
 //   * two rows of the output layer's gradient, split over the batch the same way.
 // The sums' jobs come first in the grid: they are serial chains of rows / 256 additions, a few
 // waves wide, and run beside the matrix tiles.  What bounds the launch: reading every layer's
-// input and dZ once for the tiles and once for the sums.  65536 rows: 95 us for all of it, where
+// input and dZ once for the tiles and once for the sums.  65536 rows: 107 us for all of it, where
 // a launch per layer and sum took 138 us x 4 (generic tiles), 100 us x 4 and 167 us.
 //
 // update_body finishes the sums and applies Adam to each parameter as its gradient becomes

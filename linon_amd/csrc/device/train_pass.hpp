@@ -14,9 +14,12 @@
 //     bytes a lane, 1 KB a wave), not as a row-major matrix.
 // What bounds it: at 65536 rows, 290 MB of bf16 rows and 400 MB of z to and from memory, and the
 // SiLU and its derivative (an exponential and a reciprocal each, quarter rate) beside the MFMAs.
-// 189 us there; the launches it replaces took 895 (600 of them the dX products on 2-byte loads).
+// 174 us there; the launches it replaces took 895 (600 of them the dX products on 2-byte loads).
+// Rows and z move nontemporally: as ordinary stores they push one another and the weights out of the
+// caches (185 us; the rows alone 176 and z alone 172, but then the gradients' launch that reads the
+// rows takes 112 us and not 106).
 // The weights of a layer are first read at its start: read under the layer before, as inference
-// does, they cost 190 bytes of spills more and the pass takes 217 us.
+// does, they cost 190 bytes of spills more and the pass took 217 us for 189.
 //
 // The arithmetic is that of the kernels it replaces (features_body, gemm_body's k order,
 // out_layer_kernel's and loss_kernel's expressions): the same bits.
@@ -70,8 +73,8 @@ __device__ __forceinline__ void tile_out(const u16 (*tile)[LM_FUSED_LDA], int ro
     for (int i = threadIdx.x; i < LM_FUSED_ROWS * Chunks; i += 256) {
         const int r = i / Chunks, c = i % Chunks;
         if (row0 + r < n)
-            *reinterpret_cast<u32x4v*>(out + ((size_t)(row0 + r) * Chunks + c) * 8) =
-                *reinterpret_cast<const u32x4v*>(&tile[r][c * 8]);
+            __builtin_nontemporal_store(*reinterpret_cast<const u32x4v*>(&tile[r][c * 8]),
+                                        reinterpret_cast<u32x4v*>(out + ((size_t)(row0 + r) * Chunks + c) * 8));
     }
 }
 
@@ -105,26 +108,15 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     // this thread's z scratch of layer l: 32 float4, 256 threads apart
     const size_t tiles = gridDim.x;
     auto zat = [&](int l) {
-        return reinterpret_cast<float4*>(P.z) + (((size_t)l * tiles + blockIdx.x) * 32) * 256 + tid;
+        return reinterpret_cast<f32x4v*>(P.z) + (((size_t)l * tiles + blockIdx.x) * 32) * 256 + tid;
     };
     const int nl = 64 * wave + 4 * (lane >> 5);  // this lane's columns are nl + 32 j + 8 g .. +3, its rows 32 i + lane % 32
 
     // ---- forward ----
-#pragma nounroll
-    for (int l = 0; l < 4; ++l) {
-        u32x4v wa[2][2], wb[2][2];
-        const u16* wl = P.wpack + pack_offset(l);
-        mlp_load_pair(wl, 0, wave, lane, wa);
-        if (l == 0) {
-            tile_out<LS_FEATS_PAD / 8>(tile, row0, n, P.feat);
-            mlp_layer_k<LM_FUSED_KSTEPS0, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
-        } else {
-            tile_out<LS_HIDDEN / 8>(tile, row0, n, P.act[l - 1]);
-            mlp_layer_k<LM_FUSED_KSTEPS, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
-        }
-        __syncthreads();  // every wave has read this layer's input
-        const float* bias = P.bias[l];
-        float4* z = zat(l);
+    // bias, SiLU, and the pre-activations to scratch but for the last layer's, in one straight piece
+    // each (a test at every store left pieces of 26 instructions whose exponentials had nothing to
+    // overlap with)
+    auto epilogue = [&](const float* bias, f32x4v* z, auto keep) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -138,14 +130,36 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
                     a[4 * g + 1] += bv.y;
                     a[4 * g + 2] += bv.z;
                     a[4 * g + 3] += bv.w;
-                    if (l < 3) z[((j * 4 + g) * 4 + i) * 256] = make_float4(a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]);
+                    if constexpr (!decltype(keep)::value)
+                        __builtin_nontemporal_store(f32x4v{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]},
+                                                    &z[((j * 4 + g) * 4 + i) * 256]);
                     const unsigned lo = f2bf2(silu(a[4 * g]), silu(a[4 * g + 1]));
                     const unsigned hi = f2bf2(silu(a[4 * g + 2]), silu(a[4 * g + 3]));
                     *reinterpret_cast<uint2*>(&tile[32 * i + (lane & 31)][n0]) = make_uint2(lo, hi);
                 }
             }
         __syncthreads();
+    };
+    u32x4v wa[2][2], wb[2][2];
+#pragma nounroll
+    for (int l = 0; l < 3; ++l) {
+        const u16* wl = P.wpack + pack_offset(l);
+        mlp_load_pair(wl, 0, wave, lane, wa);
+        if (l == 0) {
+            tile_out<LS_FEATS_PAD / 8>(tile, row0, n, P.feat);
+            mlp_layer_k<LM_FUSED_KSTEPS0, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
+        } else {
+            tile_out<LS_HIDDEN / 8>(tile, row0, n, P.act[l - 1]);
+            mlp_layer_k<LM_FUSED_KSTEPS, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
+        }
+        __syncthreads();  // every wave has read this layer's input
+        epilogue(P.bias[l], zat(l), IntType<0>{});
     }
+    mlp_load_pair(P.wpack + pack_offset(3), 0, wave, lane, wa);
+    tile_out<LS_HIDDEN / 8>(tile, row0, n, P.act[2]);
+    mlp_layer_k<LM_FUSED_KSTEPS, false>(P.wpack + pack_offset(3), nullptr, tile, wave, lane, acc, wa, wb);
+    __syncthreads();
+    epilogue(P.bias[3], nullptr, IntType<1>{});
 
     // ---- output layer and loss: two threads per row (outputs 0..3 and 4..6); z of the last
     // layer stays in acc ----
@@ -234,13 +248,12 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
     // ---- dZ of layer l - 1 = (dZ W^T) * silu'(z_{l-1}) ----
 #pragma nounroll
     for (int l = 3; l > 0; --l) {
-        u32x4v wa[2][2], wb[2][2];
         const u16* wl = P.bpack + (size_t)(l - 1) * LM_PACK_LAYER;
         mlp_load_pair(wl, 0, wave, lane, wa);
         tile_out<LS_HIDDEN / 8>(tile, row0, n, P.dz[l]);
         mlp_layer_k<LM_FUSED_KSTEPS, false>(wl, nullptr, tile, wave, lane, acc, wa, wb);
         __syncthreads();
-        const float4* z = zat(l - 1);
+        const f32x4v* z = zat(l - 1);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -248,7 +261,7 @@ __device__ __forceinline__ void train_pass_body(const PassParams& P) {
                 const int n0 = nl + 32 * j + 8 * g;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float4 zv = z[((j * 4 + g) * 4 + i) * 256];
+                    const f32x4v zv = __builtin_nontemporal_load(&z[((j * 4 + g) * 4 + i) * 256]);
                     const f32x16& a = acc[j][i];
                     const unsigned lo = f2bf2(a[4 * g] * silu_grad(zv.x), a[4 * g + 1] * silu_grad(zv.y));
                     const unsigned hi = f2bf2(a[4 * g + 2] * silu_grad(zv.z), a[4 * g + 3] * silu_grad(zv.w));
