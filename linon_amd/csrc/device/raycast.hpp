@@ -629,7 +629,7 @@ __device__ __forceinline__ bool ray_advance_impl(RayState& r, const StepParams& 
     return ray_finished(r, I);
 }
 
-// ray_advance_impl's loop without a mesh, fixed step, escape mode: the steps of a flow map and of
+// ray_advance_impl's loop without a mesh, fixed step, escape mode: the steps of flow maps and of
 // the approach to a surrogate's sphere, to their end.  The tests for the sphere, the stop and the
 // step cap make one condition, so that a step has one branch and one change of the lane mask (the
 // general loop has fifteen blocks and 55 scalar instructions a step without a mesh too, here 17).
@@ -662,9 +662,10 @@ __device__ __forceinline__ bool ray_advance_free(RayState& r, const StepParams& 
         step = rn::mul(r.d, h);
         q = rn::add(p, step);
         r.t = rn::add(r.t, h);
-        out = (rn::dot(q, q) > I.escape_r2) & (rn::dot(q, r.d) > 0.0f);
+        // (no && or ||: each would be a branch)
+        out = int(rn::dot(q, q) > I.escape_r2) & int(rn::dot(q, r.d) > 0.0f);
         last = r.iters >= I.max_steps;
-        return out | last | stop(q);
+        return int(out) | int(last) | int(stop(q));
     };
     // The end needs a step's start too.  Either it is copied at each step, or two steps make a pass
     // and two positions take turns: that is faster with a stop test (1080p warp approach 1.14 ms, 1.31
@@ -685,7 +686,7 @@ __device__ __forceinline__ bool ray_advance_free(RayState& r, const StepParams& 
     }
     r.p = q;
     if (out && I.clip_exit) r.p = sphere_exit(p, step, I.escape_r2);
-    return out | last;
+    return out || last;
 }
 
 template <class F, class Stop = NeverStop>

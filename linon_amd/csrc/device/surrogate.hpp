@@ -139,8 +139,8 @@ struct FlowmapParams {
 };
 
 // RK4 from an entry state to the sphere exit (the surrogate's training labels, and the
-// fallback of a frame).
-template <class F>
+// fallback of a frame).  Free: fixed steps, in the loop without a mesh; else the general loop.
+template <class F, bool Free>
 __device__ void flowmap_body(const FlowmapParams& P) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (P.n_dev ? *P.n_dev : P.n)) return;
@@ -150,7 +150,7 @@ __device__ void flowmap_body(const FlowmapParams& P) {
     lk::ray_begin(r, vec3f(s[0], s[1], s[2]), vec3f(s[3], s[4], s[5]), P.step);
     const int before = P.iters_at ? P.iters_at[P.texel_of[slot]] : 0;
     r.iters = before;
-    if (P.step.adaptive) {  // a caller's integrator
+    if constexpr (!Free) {
         SceneParams none;
         none.accel = LINON_ACCEL_BRUTE_K;
         none.num_faces = 0;

@@ -42,7 +42,12 @@ __global__ void __launch_bounds__(256) approach_kernel(ls::ApproachParams A) {
 
 template <class F>
 __global__ void __launch_bounds__(256) flowmap_kernel(ls::FlowmapParams P) {
-    ls::flowmap_body<F>(P);
+    ls::flowmap_body<F, false>(P);
+}
+
+template <class F>
+__global__ void __launch_bounds__(256) flowmap_free_kernel(ls::FlowmapParams P) {
+    ls::flowmap_body<F, true>(P);
 }
 
 // Uniform entry states: p uniform on the sphere of radius R, pulled inside by up to one step
@@ -380,23 +385,33 @@ hipError_t sg_fill_i32(int* p, int n, int value, hipStream_t s) {
     return hipGetLastError();
 }
 
-#define LS_FIELD_SWITCH(KERNEL)                                              \
-    switch (field) {                                                         \
-        case 17: return (const void*)&KERNEL<lw::FieldSwirl>;                \
-        case 18: return (const void*)&KERNEL<lw::FieldLens>;                 \
-        case 19: return (const void*)&KERNEL<lw::FieldHotAir>;               \
-        case 20: return (const void*)&KERNEL<lw::FieldWarp>;                 \
-        case LINON_KERNEL_HOT_AIR_FAITHFUL_ROOT:                             \
-            return (const void*)&KERNEL<lw::FieldHotAirFaithfulRoot>;        \
-        case LINON_KERNEL_LENS_RECIP:                                        \
-            return (const void*)&KERNEL<lw::FieldLensRecip>;                 \
-        case 3: return (const void*)&KERNEL<lw::FieldMirageSphericalSigmoid>; \
-        case 16: return (const void*)&KERNEL<lw::FieldIdentity>;             \
-        default: return nullptr;                                             \
-    }
+#define LS_FIELD_CASES(KERNEL)                                               \
+    case 17: return (const void*)&KERNEL<lw::FieldSwirl>;                    \
+    case 19: return (const void*)&KERNEL<lw::FieldHotAir>;                   \
+    case 20: return (const void*)&KERNEL<lw::FieldWarp>;                     \
+    case LINON_KERNEL_HOT_AIR_FAITHFUL_ROOT:                                 \
+        return (const void*)&KERNEL<lw::FieldHotAirFaithfulRoot>;            \
+    case 3: return (const void*)&KERNEL<lw::FieldMirageSphericalSigmoid>;    \
+    case 16: return (const void*)&KERNEL<lw::FieldIdentity>;                 \
+    default: return nullptr;
+#define LS_LENS_CASES(KERNEL)                                                \
+    case 18: return (const void*)&KERNEL<lw::FieldLens>;                     \
+    case LINON_KERNEL_LENS_RECIP:                                            \
+        return (const void*)&KERNEL<lw::FieldLensRecip>;
 
-static const void* approach_for(int field) { LS_FIELD_SWITCH(approach_kernel) }
-static const void* flowmap_for(int field) { LS_FIELD_SWITCH(flowmap_kernel) }
+static const void* approach_for(int field) {
+    switch (field) { LS_LENS_CASES(approach_kernel) LS_FIELD_CASES(approach_kernel) }
+}
+static const void* flowmap_for(int field) {
+    switch (field) { LS_LENS_CASES(flowmap_kernel) LS_FIELD_CASES(flowmap_kernel) }
+}
+// Fixed steps in the loop without a mesh: 262,144 rays with their copies hot air 2.63 -> 2.33 ms, warp
+// 1.35 -> 1.25, mirage 3.72 -> 3.41, and 3,000 rays 10-30% less.  Not the lens, whose step is mostly
+// its field's own branches: 844,000 rays take 9.12 ms so and 8.97 in the general loop, 3,000 rays
+// 1.03-1.20 and 1.16 ms a call.
+static const void* flowmap_free_for(int field) {
+    switch (field) { LS_FIELD_CASES(flowmap_free_kernel) }
+}
 
 bool sg_field_supported(int field) { return approach_for(field) != nullptr; }
 
@@ -408,7 +423,9 @@ hipError_t sg_approach(int field, const ls::ApproachParams& A, hipStream_t s) {
     return hipLaunchKernel(fn, dim3((tiles + 3) / 4), dim3(256), args, 0, s);
 }
 hipError_t sg_flowmap(int field, const ls::FlowmapParams& P, hipStream_t s) {
-    const void* fn = flowmap_for(field);
+    // adaptive steps (a caller's integrator) need the general loop
+    const void* fn = P.step.adaptive ? nullptr : flowmap_free_for(field);
+    if (!fn) fn = flowmap_for(field);
     if (!fn) return hipErrorInvalidDeviceFunction;
     if (P.n <= 0) return hipSuccess;
     void* args[] = {const_cast<ls::FlowmapParams*>(&P)};
