@@ -24,8 +24,8 @@ struct GridBuild {
 void pack_faces(const float* xyz, const uint32_t* faces, uint32_t nf, std::vector<float>& out);
 
 // Grid geometry for a mesh: bounds of the referenced vertices padded by a margin, cubic cells
-// with at most `resolution` along the longest axis.  Validates the input (indices in range,
-// finite coordinates); returns false and sets `err` otherwise.
+// `resolution` along the longest axis (one more where the rounded bounds count up).  Validates
+// the input (indices in range, finite coordinates); returns false and sets `err` otherwise.
 bool grid_geometry(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf, int resolution,
                    GridGeom& geo, std::string& err);
 

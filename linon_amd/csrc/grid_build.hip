@@ -50,7 +50,8 @@ __device__ __forceinline__ size_t range_cells(const int c0[3], const int c1[3]) 
     return (size_t)(c1[0] - c0[0] + 1) * (size_t)(c1[1] - c0[1] + 1) * (size_t)(c1[2] - c0[2] + 1);
 }
 
-// Cell k of a face's range, x fastest.  At most 1024^3 cells, so 32 bits hold every index.
+// Cell k of a face's range, x fastest.  At most 1024^3 cells, or a little more where a dimension's
+// count rounds up past the resolution: 32 bits hold every index.
 struct FaceCells {
     int x0, y0, z0;
     unsigned sx, sxy;
@@ -402,24 +403,25 @@ __global__ void __launch_bounds__(256) fill_u32_kernel(unsigned* p, size_t n, un
     if (i < n) p[i] = value;
 }
 
-constexpr int kRowChunks = 1024 / 64;  // 64-cell chunks of the longest row
-
 // Distance along x to the nearest occupied cell of the row (capped at 255), one wave per row: the
 // row's occupancy as 64-bit masks, in which every lane finds the nearest set bit on either side.
-// (A sweep of each row by one lane took 76 us for 128^3 cells, 374 us for 256^3.)
+// (A sweep of each row by one lane took 76 us for 128^3 cells, 374 us for 256^3.)  The masks are
+// sized by the launch, dist_x_lds(nx) bytes: a row can be longer than the resolution, whose cells
+// are counted up from rounded bounds (1025 for 1024 over x in [0, 0.02f]).
 __global__ void __launch_bounds__(256) dist_x_kernel(const unsigned* cell_start, int nx, size_t rows,
                                                      unsigned char* a) {
-    __shared__ unsigned long long bits[4][kRowChunks];
+    extern __shared__ unsigned long long row_masks[];
     const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
     const size_t row = (size_t)blockIdx.x * 4 + wave;
     const bool in = row < rows;
     const size_t base = row * (size_t)nx;
-    const int chunks = (nx + 63) / 64;
+    const int chunks = dist_x_chunks(nx);
+    unsigned long long* bits = row_masks + wave * chunks;
     for (int c = 0; c < chunks; ++c) {
         const int x = 64 * c + lane;
         const bool occ = in && x < nx && cell_start[base + x + 1] > cell_start[base + x];
         const unsigned long long m = __ballot(occ);
-        if (lane == 0) bits[wave][c] = m;
+        if (lane == 0) bits[c] = m;
     }
     __syncthreads();
     if (!in) return;
@@ -428,24 +430,24 @@ __global__ void __launch_bounds__(256) dist_x_kernel(const unsigned* cell_start,
         if (x >= nx) break;
         int d = 255;
         // left, the cell itself included: the highest set bit at or below it
-        unsigned long long m = bits[wave][c] & (~0ull >> (63 - lane));
+        unsigned long long m = bits[c] & (~0ull >> (63 - lane));
         for (int k = c;;) {
             if (m) {
                 d = min(d, x - (64 * k + 63 - __clzll((long long)m)));
                 break;
             }
             if (--k < 0 || x - (64 * k + 63) >= 255) break;
-            m = bits[wave][k];
+            m = bits[k];
         }
         // right: the lowest set bit at or above it
-        m = bits[wave][c] & (~0ull << lane);
+        m = bits[c] & (~0ull << lane);
         for (int k = c;;) {
             if (m) {
                 d = min(d, 64 * k + __ffsll((long long)m) - 1 - x);
                 break;
             }
             if (++k >= chunks || 64 * k - x >= 255) break;
-            m = bits[wave][k];
+            m = bits[k];
         }
         a[base + x] = (unsigned char)d;
     }
@@ -459,7 +461,7 @@ __global__ void __launch_bounds__(256) dist_minmax_kernel(const unsigned char* i
                                                           int ny, int nz, int axis) {
     const size_t cell = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= (size_t)nx * ny * nz) return;
-    const unsigned row = (unsigned)cell / (unsigned)nx;  // at most 2^30 cells
+    const unsigned row = (unsigned)cell / (unsigned)nx;  // fewer than 2^32 cells
     const int i = (int)(axis == 1 ? row % (unsigned)ny : row / (unsigned)ny);
     const int n = axis == 1 ? ny : nz;
     const size_t s = axis == 1 ? (size_t)nx : (size_t)nx * ny;
@@ -622,7 +624,7 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
             hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc + 1, 256)), dim3(256), 0, s, out.cell_start, nc + 1,
                                0u);
         }
-        hipLaunchKernelGGL(dist_x_kernel, dim3(blocks_for(ny * nz, 4)), dim3(256), 0, s,
+        hipLaunchKernelGGL(dist_x_kernel, dim3(blocks_for(ny * nz, 4)), dim3(256), dist_x_lds((int)nx), s,
                            (const unsigned*)out.cell_start, (int)nx, ny * nz, out.dist);
         hipLaunchKernelGGL(dist_minmax_kernel, dim3(blocks_for(nc, 256)), dim3(256), 0, s,
                            (const unsigned char*)out.dist, d_tmp, (int)nx, (int)ny, (int)nz, 1);

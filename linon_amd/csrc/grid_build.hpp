@@ -19,6 +19,11 @@ struct DeviceGrid {
     void release();
 };
 
+// The x pass of the distance field: 64-cell masks of a row of nx cells, and their LDS bytes for
+// a block's four rows.
+__host__ __device__ constexpr int dist_x_chunks(int nx) { return (nx + 63) / 64; }
+__host__ __device__ constexpr unsigned dist_x_lds(int nx) { return 4u * (unsigned)dist_x_chunks(nx) * 8u; }
+
 // Builds the grid of geometry `g` (from grid_geometry, which also validated the mesh) on the
 // device: uploads the mesh, counts, scans, fills, sorts and computes the distance field on
 // stream s, synchronising twice.  On failure returns false with `err` set and nothing allocated.

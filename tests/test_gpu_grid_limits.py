@@ -1,0 +1,45 @@
+"""The device grid build where its sizes and its memory end, against the host build."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import linon_amd as L
+
+pytestmark = pytest.mark.gpu
+
+
+def same_grids(view):
+    view.set_grid_builder(L.GRID_BUILD_HOST)
+    h = view.read_grid()
+    view.set_grid_builder(L.GRID_BUILD_DEVICE)
+    d = view.read_grid()
+    for k in ("dims", "cell_start", "cell_faces", "dist", "tris"):
+        np.testing.assert_array_equal(h[k], d[k], err_msg=k)
+    return d
+
+
+def small_faces(n, size, at, seed):
+    rng = np.random.default_rng(seed)
+    c = at(rng, n)[:, None, :] + size * rng.uniform(-1.0, 1.0, (n, 3, 3))
+    return c.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+
+def test_rows_longer_than_the_resolution():
+    """Over x in [0, 0.02f] a resolution of 1024 makes 1025 cells: 17 masks of 64 cells a row.  Faces in
+    the first 64 cells of some rows, in the last of others, in most none; y and z stay narrow."""
+    def at(rng, n):
+        x = np.where(rng.random(n) < 0.5, rng.uniform(0.0002, 0.001, n), rng.uniform(0.019, 0.0198, n))
+        return np.stack([x, rng.uniform(0.0, 4e-4, n), rng.uniform(0.0, 4e-4, n)], 1)
+    v, f = small_faces(60, 1e-5, at, 3)
+    v = np.concatenate([v, np.array([[0, 0, 0], [0.02, 0, 0], [0.02, 1e-5, 0]], np.float32)])
+    f = np.concatenate([f, [[180, 180, 180], [181, 182, 181]]]).astype(np.uint32)
+    print("[case] grid build, a row of 1025 cells", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_grid_builder(L.GRID_BUILD_HOST)
+        view.set_accel(L.ACCEL_GRID, 1024)
+        view.update_model(v, f)
+        d = same_grids(view)
+    assert d["dims"][0] == 1025
+    occupied = np.diff(d["cell_start"]).reshape(d["dims"][::-1]) > 0
+    assert occupied[..., :64].any() and occupied[..., 960:].any()

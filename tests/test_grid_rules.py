@@ -1,0 +1,48 @@
+"""CPU checks of the rules the grid builds go by (grid.cpp and grid_build.hpp, built with g++)."""
+from __future__ import annotations
+
+import ctypes as C
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+CSRC = ROOT / "linon_amd" / "csrc"
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = tmp_path_factory.mktemp("grid") / "grid_shim.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{CSRC}", str(ROOT / "tests" / "host" / "grid_shim.cpp"), str(CSRC / "grid.cpp"), "-pthread",
+                    "-o", str(so)], check=True)
+    return C.CDLL(str(so))
+
+
+def arrays(v, f):
+    v = np.ascontiguousarray(v, np.float32).reshape(-1, 3)
+    f = np.ascontiguousarray(f, np.uint32).reshape(-1, 3)
+    return v, f, (v.ctypes.data_as(C.c_void_p), len(v), f.ctypes.data_as(C.c_void_p), len(f))
+
+
+def flat(x, y=0.01):
+    return np.array([[0, 0, 0], [x, 0, 0], [x, y * x, 0]], np.float32), np.array([[0, 1, 2]], np.uint32)
+
+
+def test_row_masks_hold_the_longest_row(lib):
+    """The cells of a dimension are counted up from rounded bounds, so a row can hold more cells than
+    the resolution; the masks of a row have a bit for each."""
+    longest = 0
+    for x in (np.float32(0.02), *np.random.default_rng(0).uniform(1e-3, 1.0, 500)):
+        v, f, args = arrays(*flat(x))
+        dims = (C.c_int * 3)()
+        assert lib.grid_dims(*args, 1024, dims)
+        longest = max(longest, dims[0])
+        assert 64 * lib.row_mask_chunks(dims[0]) >= dims[0]
+        assert lib.row_mask_bytes(dims[0]) == 4 * 8 * lib.row_mask_chunks(dims[0]) <= 65536
+    assert longest == 1025
