@@ -243,6 +243,9 @@ typedef enum linon_grid_builder {
     LINON_GRID_BUILD_DEVICE = 2
 } linon_grid_builder;
 linon_status linon_set_grid_builder(linon_context* ctx, int builder);
+/* Diagnostics (for tests of full device memory; no counterpart in the reference): allocation
+ * `number`, 1 to 6, of each following device build of the context's grid is refused; 0: none. */
+linon_status linon_selftest_refuse_grid_alloc(linon_context* ctx, int number);
 /* The grid of the current mesh (for tests; no counterpart in the reference): dims[3], the
  * ncells + 1 cell offsets, the face ids of every cell, the ncells distance bytes, the packed
  * faces (12 floats each) and the reference count.  Null pointers skip an array; sizes are

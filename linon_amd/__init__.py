@@ -233,6 +233,7 @@ SIGNATURES = {
     "linon_set_mesh": (C.c_int, [_P, _P, C.c_uint32, _P, C.c_uint32]),
     "linon_set_accel": (C.c_int, [_P, C.c_int, C.c_int]),
     "linon_set_grid_builder": (C.c_int, [_P, C.c_int]),
+    "linon_selftest_refuse_grid_alloc": (C.c_int, [_P, C.c_int]),
     "linon_set_math": (C.c_int, [_P, C.c_int]),
     "linon_selftest_division": (C.c_int, [C.c_int, C.c_uint64, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64),
                                           C.POINTER(C.c_uint64)]),

@@ -307,7 +307,7 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
         LN_CHECK_HIP(this, hipDeviceSynchronize());
         free_mesh();
         DeviceGrid dg;
-        if (build_grid_device(geo, h_xyz.data(), nv, h_faces.data(), nf, stream, dg, e)) {
+        if (build_grid_device(geo, h_xyz.data(), nv, h_faces.data(), nf, stream, grid_refuse_alloc, dg, e)) {
             d_tris = dg.tris;
             d_cell_start = dg.cell_start;
             d_cell_faces = dg.cell_faces;
@@ -606,6 +606,15 @@ linon_status linon_set_grid_builder(linon_context* ctx, int builder) {
     c->grid_builder = builder;
     if (rebuild) return c->upload_mesh(c->h_xyz.data(), (uint32_t)(c->h_xyz.size() / 3), c->h_faces.data(),
                                        (uint32_t)(c->h_faces.size() / 3));
+    return LINON_OK;
+}
+
+linon_status linon_selftest_refuse_grid_alloc(linon_context* ctx, int number) {
+    Context* c = reinterpret_cast<Context*>(ctx);
+    LN_CTX(c);
+    if (number < 0 || number > linon::GRID_BUILD_ALLOCS)
+        return c->fail(LINON_ERR_ARGUMENT, "selftest_refuse_grid_alloc: no allocation of that number");
+    c->grid_refuse_alloc = number;
     return LINON_OK;
 }
 

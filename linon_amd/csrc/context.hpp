@@ -146,6 +146,7 @@ struct Context {
     int grid_res_req = 0;
     int grid_builder = LINON_GRID_BUILD_AUTO;
     bool grid_on_device = false;  // how the current grid was built
+    int grid_refuse_alloc = 0;    // linon_selftest_refuse_grid_alloc
     std::vector<float> h_xyz;
     std::vector<uint32_t> h_faces;
 

@@ -516,7 +516,10 @@ struct Arena {
         bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
         return (int)at.size() - 1;
     }
-    hipError_t allocate() { return hipMalloc(&base, bytes); }
+    template <class Alloc>
+    hipError_t allocate(Alloc& alloc) {
+        return alloc(&base, bytes);
+    }
     template <class T>
     T* get(int i) const {
         return reinterpret_cast<T*>(base + at[(size_t)i]);
@@ -529,7 +532,7 @@ struct Arena {
 }  // namespace
 
 bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
-                       hipStream_t s, DeviceGrid& out, std::string& err) {
+                       hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err) {
     out.release();
     const size_t nx = (size_t)g.dim[0], ny = (size_t)g.dim[1], nz = (size_t)g.dim[2];
     const size_t nc = nx * ny * nz;
@@ -546,10 +549,14 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
         if (e != hipSuccess) err = std::string("device grid build: ") + what + ": " + hipGetErrorString(e);
         return e == hipSuccess;
     };
+    int allocs = 0;
+    auto alloc = [&](auto** p, size_t bytes) {
+        return hipMalloc(p, ++allocs == refuse_alloc ? size_t{1} << 50 : bytes);
+    };
     auto build = [&]() {
-        if (!check(A.allocate(), "alloc") || !check(hipMalloc(&out.cell_start, (nc + 1) * 4), "alloc") ||
-            !check(hipMalloc(&out.dist, nc), "alloc") ||
-            !check(hipMalloc(&out.tris, std::max<size_t>(1, (size_t)nf) * 48), "alloc"))
+        if (!check(A.allocate(alloc), "alloc") || !check(alloc(&out.cell_start, (nc + 1) * 4), "alloc") ||
+            !check(alloc(&out.dist, nc), "alloc") ||
+            !check(alloc(&out.tris, std::max<size_t>(1, (size_t)nf) * 48), "alloc"))
             return false;
         float* d_xyz = A.get<float>(i_xyz);
         uint32_t* d_faces = A.get<uint32_t>(i_faces);
@@ -600,10 +607,10 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
             }
         }
         const int i_refs = R.add<Reference>((size_t)total), i_list = R.add<unsigned>((size_t)total);
-        if (!check(hipMalloc(&out.cell_faces, std::max<size_t>(1, (size_t)total) * 4), "alloc")) return false;
+        if (!check(alloc(&out.cell_faces, std::max<size_t>(1, (size_t)total) * 4), "alloc")) return false;
         out.refs = (size_t)total;
         if (total) {
-            if (!check(R.allocate(), "alloc")) return false;
+            if (!check(R.allocate(alloc), "alloc")) return false;
             Reference* d_refs = R.get<Reference>(i_refs);
             unsigned* d_list = R.get<unsigned>(i_list);
             hipLaunchKernelGGL(face_place_kernel, dim3(face_blocks), dim3(256), 0, s, g, d_xyz, d_faces, nf,
@@ -637,6 +644,7 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
     if (!ok) {
         (void)hipStreamSynchronize(s);  // nothing may still run on what is freed
         out.release();
+        (void)hipGetLastError();  // it has been reported: the next launch's check must not find it
     }
     return ok;
 }

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import linon_amd as L
+from linon_amd import scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +44,36 @@ def test_rows_longer_than_the_resolution():
     assert d["dims"][0] == 1025
     occupied = np.diff(d["cell_start"]).reshape(d["dims"][::-1]) > 0
     assert occupied[..., :64].any() and occupied[..., 960:].any()
+
+
+def refuse(view, number):
+    view._check(view._lib.linon_selftest_refuse_grid_alloc(view._h, number))
+
+
+def train_one_step(view):
+    view.train_surrogate(L.SurrogateConfig.make("swirl", steps=1, train_rays=2048, batch=256, lr=1e-3, h=0.01,
+                                                max_steps=200, tolerance=1e-4, seed=1))
+
+
+@pytest.mark.parametrize("number", range(1, 7))
+def test_no_room_for_the_device_build(number):
+    """Each of the build's allocations refused in turn: AUTO has the host's arrays, and the calls that
+    follow know nothing of it."""
+    v, f = scenes.benchmark_scene(level=3)
+    print(f"[case] grid build without its allocation {number}", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_grid_builder(L.GRID_BUILD_HOST)
+        view.update_model(v, f)
+        h = view.read_grid()
+        refuse(view, number)
+        view.set_grid_builder(L.GRID_BUILD_AUTO)
+        a = view.read_grid()
+        for k in h:
+            np.testing.assert_array_equal(a[k], h[k], err_msg=k)
+        train_one_step(view)
+        with pytest.raises(L.LinonError, match="out of memory"):
+            view.set_grid_builder(L.GRID_BUILD_DEVICE)
+        train_one_step(view)
+        refuse(view, 0)
+        view.update_model(v, f)
+        same_grids(view)
