@@ -534,6 +534,7 @@ struct Arena {
 bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
                        hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err) {
     out.release();
+    (void)hipGetLastError();  // an earlier call's error is not this build's: its launches are checked below
     const size_t nx = (size_t)g.dim[0], ny = (size_t)g.dim[1], nz = (size_t)g.dim[2];
     const size_t nc = nx * ny * nz;
     const size_t longest = std::max<size_t>(nc, nf);

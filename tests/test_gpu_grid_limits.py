@@ -1,6 +1,8 @@
 """The device grid build where its sizes and its memory end, against the host build."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -75,5 +77,17 @@ def test_no_room_for_the_device_build(number):
             view.set_grid_builder(L.GRID_BUILD_DEVICE)
         train_one_step(view)
         refuse(view, 0)
+        view.update_model(v, f)
+        same_grids(view)
+
+
+def test_an_earlier_error_is_not_the_builds():
+    """An error that another call on this thread left unread: the device build succeeds all the same."""
+    v, f = scenes.benchmark_scene(level=2)
+    print("[case] grid build after another call's error", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_grid_builder(L.GRID_BUILD_DEVICE)
+        p = C.c_void_p()
+        assert view._lib.hipMalloc(C.byref(p), C.c_size_t(1 << 50)) == 2  # hipErrorOutOfMemory
         view.update_model(v, f)
         same_grids(view)
