@@ -307,7 +307,9 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
         LN_CHECK_HIP(this, hipDeviceSynchronize());
         free_mesh();
         DeviceGrid dg;
-        if (build_grid_device(geo, h_xyz.data(), nv, h_faces.data(), nf, stream, grid_refuse_alloc, dg, e)) {
+        const GridResult r =
+            build_grid_device(geo, h_xyz.data(), nv, h_faces.data(), nf, stream, grid_refuse_alloc, dg, e);
+        if (r == GridResult::BUILT) {
             d_tris = dg.tris;
             d_cell_start = dg.cell_start;
             d_cell_faces = dg.cell_faces;
@@ -325,7 +327,11 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
             grid_on_device = true;
             return batch.d_views ? batch_capture() : LINON_OK;
         }
-        if (grid_builder == LINON_GRID_BUILD_DEVICE) return fail(LINON_ERR_HIP, "set_mesh: " + e);
+        // the host's verdict on the references would be the same, after gathering 32 GB of them
+        if (grid_builder == LINON_GRID_BUILD_DEVICE || r != GridResult::NO_ROOM)
+            return fail(r == GridResult::TOO_LARGE && grid_builder == LINON_GRID_BUILD_AUTO ? LINON_ERR_ARGUMENT
+                                                                                            : LINON_ERR_HIP,
+                        "set_mesh: " + e);
         xyz = h_xyz.data();
         faces = h_faces.data();
     }

@@ -531,7 +531,7 @@ struct Arena {
 
 }  // namespace
 
-bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
+GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
                        hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err) {
     out.release();
     (void)hipGetLastError();  // an earlier call's error is not this build's: its launches are checked below
@@ -546,9 +546,12 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
     const int i_cursor = A.add<unsigned>(nf), i_cells = A.add<unsigned>(nc);
     const int i_local = A.add<unsigned long long>(longest), i_bsum = A.add<unsigned long long>(max_blocks);
     const int i_total = A.add<unsigned long long>(1), i_nbig = A.add<unsigned>(2), i_tmp = A.add<unsigned char>(nc);
+    GridResult result = GridResult::BUILT;
     auto check = [&](hipError_t e, const char* what) {
-        if (e != hipSuccess) err = std::string("device grid build: ") + what + ": " + hipGetErrorString(e);
-        return e == hipSuccess;
+        if (e == hipSuccess) return true;
+        err = std::string("device grid build: ") + what + ": " + hipGetErrorString(e);
+        result = e == hipErrorOutOfMemory ? GridResult::NO_ROOM : GridResult::FAILED;
+        return false;
     };
     int allocs = 0;
     auto alloc = [&](auto** p, size_t bytes) {
@@ -604,6 +607,7 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
                 return false;
             if (total > 0xFFFFFFFFull) {
                 err = "grid has more than 2^32 face references; lower the resolution";
+                result = GridResult::TOO_LARGE;
                 return false;
             }
         }
@@ -641,13 +645,12 @@ bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const
         return check(hipGetLastError(), "place/distance launch") &&
                check(hipStreamSynchronize(s), "place/distance");
     };
-    const bool ok = build();
-    if (!ok) {
+    if (!build()) {
         (void)hipStreamSynchronize(s);  // nothing may still run on what is freed
         out.release();
         (void)hipGetLastError();  // it has been reported: the next launch's check must not find it
     }
-    return ok;
+    return result;
 }
 
 }  // namespace linon

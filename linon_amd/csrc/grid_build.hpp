@@ -26,11 +26,17 @@ __host__ __device__ constexpr unsigned dist_x_lds(int nx) { return 4u * (unsigne
 
 // Builds the grid of geometry `g` (from grid_geometry, which also validated the mesh) on the
 // device: uploads the mesh, counts, scans, fills, sorts and computes the distance field on
-// stream s, synchronising twice.  On failure returns false with `err` set and nothing allocated.
+// stream s, synchronising twice.  On failure `err` is set and nothing is allocated.
 // `refuse_alloc` > 0: the build's allocation of that number asks for a petabyte (tests of full
 // memory); a build makes GRID_BUILD_ALLOCS of them.
 constexpr int GRID_BUILD_ALLOCS = 6;
-bool build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
+enum class GridResult {
+    BUILT,
+    NO_ROOM,    // the device has no memory for the grid or the build's scratch
+    TOO_LARGE,  // more references than a grid holds
+    FAILED      // any other error of HIP's
+};
+GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
                        hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err);
 
 }  // namespace linon

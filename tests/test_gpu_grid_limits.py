@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -90,4 +91,26 @@ def test_an_earlier_error_is_not_the_builds():
         p = C.c_void_p()
         assert view._lib.hipMalloc(C.byref(p), C.c_size_t(1 << 50)) == 2  # hipErrorOutOfMemory
         view.update_model(v, f)
+        same_grids(view)
+
+
+def too_many_references():
+    """Faces of half the cells of a flat 1024 x 1024 grid each, more than 2^32 references in all."""
+    v = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0]], np.float32)
+    return v, np.tile(np.array([[0, 1, 2]], np.uint32), (9000, 1))
+
+
+@pytest.mark.parametrize("builder, status", [(L.GRID_BUILD_AUTO, "ARGUMENT"), (L.GRID_BUILD_DEVICE, "HIP")])
+def test_too_many_references_are_refused_at_once(builder, status):
+    """By the device's count alone: the host would gather them all first, 34 GB."""
+    v, f = too_many_references()
+    print(f"[case] grid of more than 2^32 references, builder {builder}", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_accel(L.ACCEL_GRID, 1024)
+        view.set_grid_builder(builder)
+        t = time.perf_counter()
+        with pytest.raises(L.LinonError, match=f"{status}.*2\\^32 face references"):
+            view.update_model(v, f)
+        assert time.perf_counter() - t < 30.0
+        view.update_model(v, f[:1])
         same_grids(view)
