@@ -301,15 +301,35 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
         GridGeom geo;
         std::string e;
         if (!grid_geometry(xyz, nv, faces, nf, res, geo, e)) return fail(LINON_ERR_ARGUMENT, "set_mesh: " + e);
-        if (h_xyz.data() != xyz) h_xyz.assign(xyz, xyz + 3 * (size_t)nv);
-        if (h_faces.data() != faces) h_faces.assign(faces, faces + 3 * (size_t)nf);
+        // host copies: a later linon_set_accel may rebuild the grid (from them)
+        const bool own = h_xyz.data() == xyz && h_faces.data() == faces;
+        std::vector<float> new_xyz;
+        std::vector<uint32_t> new_faces;
+        if (!own) {
+            new_xyz.assign(xyz, xyz + 3 * (size_t)nv);
+            new_faces.assign(faces, faces + 3 * (size_t)nf);
+        }
         LN_CHECK_HIP(this, hipSetDevice(device));
-        LN_CHECK_HIP(this, hipDeviceSynchronize());
-        free_mesh();
         DeviceGrid dg;
-        const GridResult r =
-            build_grid_device(geo, h_xyz.data(), nv, h_faces.data(), nf, stream, grid_refuse_alloc, dg, e);
+        GridResult r = build_grid_device(geo, xyz, nv, faces, nf, stream, grid_refuse_alloc, dg, e);
+        // the present mesh stays until the new one is built (a refused one leaves it as it was),
+        // unless the two do not fit together
+        if (r == GridResult::NO_ROOM && have_mesh) {
+            LN_CHECK_HIP(this, hipDeviceSynchronize());
+            free_mesh();
+            r = build_grid_device(geo, xyz, nv, faces, nf, stream, grid_refuse_alloc, dg, e);
+        }
         if (r == GridResult::BUILT) {
+            const hipError_t idle = hipDeviceSynchronize();  // no render still reads the present one
+            if (idle != hipSuccess) {
+                dg.release();
+                LN_CHECK_HIP(this, idle);
+            }
+            free_mesh();
+            if (!own) {
+                h_xyz.swap(new_xyz);
+                h_faces.swap(new_faces);
+            }
             d_tris = dg.tris;
             d_cell_start = dg.cell_start;
             d_cell_faces = dg.cell_faces;
@@ -332,8 +352,6 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
             return fail(r == GridResult::TOO_LARGE && grid_builder == LINON_GRID_BUILD_AUTO ? LINON_ERR_ARGUMENT
                                                                                             : LINON_ERR_HIP,
                         "set_mesh: " + e);
-        xyz = h_xyz.data();
-        faces = h_faces.data();
     }
     GridBuild g;
     std::string e;

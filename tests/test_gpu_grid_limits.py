@@ -114,3 +114,29 @@ def test_too_many_references_are_refused_at_once(builder, status):
         assert time.perf_counter() - t < 30.0
         view.update_model(v, f[:1])
         same_grids(view)
+
+
+@pytest.mark.parametrize("builder", [L.GRID_BUILD_AUTO, L.GRID_BUILD_DEVICE])
+def test_a_refused_mesh_leaves_the_present_one(builder):
+    v, f = too_many_references()
+    print(f"[case] a mesh refused beside another, builder {builder}", flush=True)
+    with L.MainView(32, 24) as view:
+        view.set_accel(L.ACCEL_GRID, 1024)
+        view.set_grid_builder(builder)
+        view.update_model(v, f[:3])
+        view.update_camera(L.Camera.look_at((0.3, 0.3, 1.0), (0.3, 0.3, 0.0), (0.0, 1.0, 0.0), fov_deg=60.0))
+        view.set_integrator(L.Integrator.make(h_initial=0.1, adaptive=False, samples_per_ray=0, sample_steps=0))
+        view.set_field("identity")
+        view.render()
+        want, grid = view.read_hit_faces(), view.read_grid()
+        assert (want >= 0).any()
+        with pytest.raises(L.LinonError, match="face references"):
+            view.update_model(v, f)
+        got = view.read_grid()
+        for k in grid:
+            np.testing.assert_array_equal(got[k], grid[k], err_msg=k)
+        view.render()
+        np.testing.assert_array_equal(view.read_hit_faces(), want)
+        view.set_accel(L.ACCEL_GRID, 64)   # rebuilt from the context's own copy of the mesh
+        view.render()
+        assert (view.read_hit_faces() >= 0).any()
