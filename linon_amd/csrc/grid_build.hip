@@ -196,32 +196,33 @@ __global__ void __launch_bounds__(1024) classify_kernel(GridGeom g, const float*
 // up to 256 cells one after another (0.5 ms, twice: the second time to place them).
 __global__ void __launch_bounds__(256) face_overlap_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
                                                            uint32_t nf, unsigned short* masks, unsigned* count) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t f = t / kFaceLanes;
-    const unsigned sub = (unsigned)t % kFaceLanes;
-    if (f >= nf) return;
-    double v[3][3];
-    load_face(xyz, faces, (uint32_t)f, v);
-    int c0[3], c1[3];
-    face_cell_range(g, v, c0, c1);
-    unsigned mask = 0;
-    // (an empty range, outside the grid, cannot happen: the grid encloses every face)
-    if (c1[0] >= c0[0] && c1[1] >= c0[1] && c1[2] >= c0[2]) {
-        const size_t cells = range_cells(c0, c1);
-        if (cells <= kMidFaceCells) {
-            const FaceCells C(c0, c1);
-            const FaceTest T(g, v);
-            int x, y, z;
-            for (unsigned k = sub, i = 0; k < (unsigned)cells; k += kFaceLanes, ++i) {
-                C.at(k, x, y, z);
-                if (T.in_cell(g, v, x, y, z)) mask |= 1u << i;
+    const unsigned sub = threadIdx.x % kFaceLanes;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < (size_t)nf * kFaceLanes; t += stride) {
+        const size_t f = t / kFaceLanes;
+        double v[3][3];
+        load_face(xyz, faces, (uint32_t)f, v);
+        int c0[3], c1[3];
+        face_cell_range(g, v, c0, c1);
+        unsigned mask = 0;
+        // (an empty range, outside the grid, cannot happen: the grid encloses every face)
+        if (c1[0] >= c0[0] && c1[1] >= c0[1] && c1[2] >= c0[2]) {
+            const size_t cells = range_cells(c0, c1);
+            if (cells <= kMidFaceCells) {
+                const FaceCells C(c0, c1);
+                const FaceTest T(g, v);
+                int x, y, z;
+                for (unsigned k = sub, i = 0; k < (unsigned)cells; k += kFaceLanes, ++i) {
+                    C.at(k, x, y, z);
+                    if (T.in_cell(g, v, x, y, z)) mask |= 1u << i;
+                }
             }
         }
+        masks[t] = (unsigned short)mask;
+        unsigned n = (unsigned)__popc(mask);
+        for (int off = kFaceLanes / 2; off > 0; off >>= 1) n += __shfl_xor(n, off, kFaceLanes);
+        if (sub == 0) count[f] = n;  // 0 for a listed face: its own kernel adds its references
     }
-    masks[t] = (unsigned short)mask;
-    unsigned n = (unsigned)__popc(mask);
-    for (int off = kFaceLanes / 2; off > 0; off >>= 1) n += __shfl_xor(n, off, kFaceLanes);
-    if (sub == 0) count[f] = n;  // 0 for a listed face: its own kernel adds its references
 }
 
 // A reference's slot in its cell.
@@ -233,28 +234,29 @@ __device__ __forceinline__ Reference take_slot(unsigned cell, unsigned face, uns
 __global__ void __launch_bounds__(256) face_place_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
                                                          uint32_t nf, const unsigned short* masks,
                                                          const unsigned* first, unsigned* cell_count, Reference* refs) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t f = t / kFaceLanes;
-    const unsigned sub = (unsigned)t % kFaceLanes;
-    if (f >= nf) return;
-    unsigned mask = masks[t];
-    const unsigned n = (unsigned)__popc(mask);
-    unsigned upto = n;  // inclusive prefix over the face's lanes
-    for (unsigned off = 1; off < (unsigned)kFaceLanes; off <<= 1) {
-        const unsigned x = __shfl_up(upto, off, kFaceLanes);
-        if (sub >= off) upto += x;
-    }
-    if (!mask) return;
-    double v[3][3];
-    load_face(xyz, faces, (uint32_t)f, v);
-    int c0[3], c1[3];
-    face_cell_range(g, v, c0, c1);
-    const FaceCells C(c0, c1);
-    Reference* out = refs + first[f] + (upto - n);
-    int x, y, z;
-    for (; mask; mask &= mask - 1) {
-        C.at(sub + kFaceLanes * (unsigned)(__ffs((int)mask) - 1), x, y, z);
-        *out++ = take_slot(cell_index(g, x, y, z), (unsigned)f, cell_count);
+    const unsigned sub = threadIdx.x % kFaceLanes;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < (size_t)nf * kFaceLanes; t += stride) {
+        const size_t f = t / kFaceLanes;
+        unsigned mask = masks[t];
+        const unsigned n = (unsigned)__popc(mask);
+        unsigned upto = n;  // inclusive prefix over the face's lanes
+        for (unsigned off = 1; off < (unsigned)kFaceLanes; off <<= 1) {
+            const unsigned x = __shfl_up(upto, off, kFaceLanes);
+            if (sub >= off) upto += x;
+        }
+        if (!mask) continue;
+        double v[3][3];
+        load_face(xyz, faces, (uint32_t)f, v);
+        int c0[3], c1[3];
+        face_cell_range(g, v, c0, c1);
+        const FaceCells C(c0, c1);
+        Reference* out = refs + first[f] + (upto - n);
+        int x, y, z;
+        for (; mask; mask &= mask - 1) {
+            C.at(sub + kFaceLanes * (unsigned)(__ffs((int)mask) - 1), x, y, z);
+            *out++ = take_slot(cell_index(g, x, y, z), (unsigned)f, cell_count);
+        }
     }
 }
 
@@ -320,10 +322,10 @@ __global__ void __launch_bounds__(256) big_overlap_kernel(GridGeom g, const floa
 // Each reference to its slot of its cell's list.
 __global__ void __launch_bounds__(256) list_kernel(const Reference* refs, size_t n, const unsigned* cell_start,
                                                    unsigned* list) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const Reference r = refs[i];
-    list[(size_t)cell_start[r.cell] + r.slot] = r.face;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        const Reference r = refs[i];
+        list[(size_t)cell_start[r.cell] + r.slot] = r.face;
+    }
 }
 
 // Each reference to its rank in its cell: the ascending order of the face ids (distinct in a
@@ -332,13 +334,13 @@ __global__ void __launch_bounds__(256) list_kernel(const Reference* refs, size_t
 // for 1.3 M faces in 256^3 cells).
 __global__ void __launch_bounds__(256) rank_kernel(const Reference* refs, size_t n, const unsigned* cell_start,
                                                    const unsigned* list, unsigned* cell_faces) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const Reference r = refs[i];
-    const unsigned b = cell_start[r.cell], e = cell_start[r.cell + 1];
-    unsigned rank = 0;
-    for (unsigned j = b; j < e; ++j) rank += list[j] < r.face ? 1u : 0u;
-    cell_faces[(size_t)b + rank] = r.face;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        const Reference r = refs[i];
+        const unsigned b = cell_start[r.cell], e = cell_start[r.cell + 1];
+        unsigned rank = 0;
+        for (unsigned j = b; j < e; ++j) rank += list[j] < r.face ? 1u : 0u;
+        cell_faces[(size_t)b + rank] = r.face;
+    }
 }
 
 __device__ __forceinline__ unsigned long long block_inclusive_scan(unsigned long long v, unsigned long long* s) {
@@ -582,7 +584,7 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
         unsigned long long total = 0;
         const dim3 mid_grid((unsigned)std::max<size_t>(1, std::min<size_t>(((size_t)nf + 3) / 4, 4096)));
         const dim3 huge_grid((unsigned)std::max<size_t>(1, std::min<size_t>(nf, 64)), 64);
-        const unsigned face_blocks = blocks_for((size_t)nf * kFaceLanes, 256);
+        const unsigned face_blocks = stride_blocks((size_t)nf * kFaceLanes);
         if (nf) {
             if (nv && !check(hipMemcpyAsync(d_xyz, h_xyz, 3 * (size_t)nv * 4, hipMemcpyHostToDevice, s), "upload"))
                 return false;
@@ -625,11 +627,11 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
             big_overlap_kernel<true, true><<<huge_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, nullptr,
                                                                      d_first, d_cursor, d_cells, d_refs);
             scan(d_cells, nc, out.cell_start);
-            hipLaunchKernelGGL(list_kernel, dim3(blocks_for((size_t)total, 256)), dim3(256), 0, s,
+            hipLaunchKernelGGL(list_kernel, dim3(stride_blocks((size_t)total)), dim3(256), 0, s,
                                (const Reference*)d_refs, (size_t)total, (const unsigned*)out.cell_start, d_list);
             hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, out.cell_start + nc, (size_t)1,
                                (unsigned)total);
-            hipLaunchKernelGGL(rank_kernel, dim3(blocks_for((size_t)total, 256)), dim3(256), 0, s,
+            hipLaunchKernelGGL(rank_kernel, dim3(stride_blocks((size_t)total)), dim3(256), 0, s,
                                (const Reference*)d_refs, (size_t)total, (const unsigned*)out.cell_start,
                                (const unsigned*)d_list, out.cell_faces);
         } else {

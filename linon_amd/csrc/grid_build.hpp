@@ -24,6 +24,13 @@ struct DeviceGrid {
 __host__ __device__ constexpr int dist_x_chunks(int nx) { return (nx + 63) / 64; }
 __host__ __device__ constexpr unsigned dist_x_lds(int nx) { return 4u * (unsigned)dist_x_chunks(nx) * 8u; }
 
+// Blocks of 256 lanes for the kernels with 16 lanes a face or a lane a reference, which stride over
+// what is left: a launch holds fewer than 2^32 lanes, 2^28 faces' worth, and 16,384 blocks are
+// eight times what the device runs at once.
+constexpr unsigned stride_blocks(size_t lanes) {
+    return (unsigned)(lanes < (size_t{1} << 22) ? (lanes + 255) / 256 : size_t{1} << 14);
+}
+
 // Builds the grid of geometry `g` (from grid_geometry, which also validated the mesh) on the
 // device: uploads the mesh, counts, scans, fills, sorts and computes the distance field on
 // stream s, synchronising twice.  On failure `err` is set and nothing is allocated.

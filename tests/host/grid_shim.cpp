@@ -16,4 +16,5 @@ int grid_dims(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf,
 
 int row_mask_chunks(int nx) { return linon::dist_x_chunks(nx); }
 unsigned row_mask_bytes(int nx) { return linon::dist_x_lds(nx); }
+unsigned stride_blocks(size_t lanes) { return linon::stride_blocks(lanes); }
 }

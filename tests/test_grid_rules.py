@@ -46,3 +46,12 @@ def test_row_masks_hold_the_longest_row(lib):
         assert 64 * lib.row_mask_chunks(dims[0]) >= dims[0]
         assert lib.row_mask_bytes(dims[0]) == 4 * 8 * lib.row_mask_chunks(dims[0]) <= 65536
     assert longest == 1025
+
+
+def test_no_launch_has_too_many_lanes(lib):
+    """A launch holds fewer than 2^32 lanes.  16 lanes a face at 2^28 faces, and a lane a reference at
+    2^32 - 1 references, are as many and more; small ones get a lane each."""
+    for lanes in (16 << 28, 16 * (2**32 // 3), 2**32 - 1, (1 << 22) - 1, 1 << 22):
+        assert lib.stride_blocks(C.c_size_t(lanes)) * 256 < 2**32
+    for lanes in (1, 16, 256, 257, 16 * 20516, (1 << 22) - 1):
+        assert lanes <= lib.stride_blocks(C.c_size_t(lanes)) * 256 < lanes + 256
