@@ -340,6 +340,8 @@ hipError_t sg_reduce(const float* part, int splits, int n, float* out, hipStream
     return hipGetLastError();
 }
 hipError_t sg_grads(const lm::GradParams& P, hipStream_t s) {
+    for (const lm::GemmParams& dw : P.dw)  // the tiles read whole steps only, and know no other loop
+        if (!lm::gemm_tn_applies(dw)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(grads_kernel, dim3(lm::grads_sum_blocks() + lm::grads_tiles(P)), dim3(256), 0, s, P);
     return hipGetLastError();
 }

@@ -123,3 +123,19 @@ def test_first_training_step(batch):
         # the padding rows of the first layer have no gradient and stay
         if k == 0:
             assert np.array_equal(b[198:], a[198:])
+
+
+# the sums' unrolled pieces: 8 rows and one more; 16 rows for some of the 256 sums and not for others;
+# 18 chunks, so that the update adds 16 partials and two single ones
+@pytest.mark.parametrize("batch", [2112, 4160, 17472])
+def test_first_step_of_a_large_batch(batch):
+    test_first_training_step(batch)
+
+
+@pytest.mark.parametrize("batch", [0, 255, 288, 1056])
+def test_batches_of_other_than_whole_chunks_are_refused(batch):
+    """The gradient tiles read whole steps of 32 rows of chunks that end with the batch."""
+    with L.MainView(16, 16) as view:
+        with pytest.raises(L.LinonError, match="bad configuration"):
+            view.train_surrogate(L.SurrogateConfig.make("swirl", steps=1, train_rays=2048, batch=batch, lr=1e-3,
+                                                        h=0.01, max_steps=1000, tolerance=1e-4, seed=7))
