@@ -10,7 +10,6 @@
 
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -105,8 +104,9 @@ hipError_t ReadStaging::copy(const HostCopy* copies, int n, hipStream_t stream, 
     try {
         for (; started < THREADS - 1 && (size_t)started + 1 < chunks_all; ++started)
             pool[started] = std::thread(work, started + 1);
-    } catch (const std::system_error&) {
-        // no more threads to be had: those started, and this one, do the work
+    } catch (...) {
+        // no more threads to be had (std::system_error), or no memory for one (std::bad_alloc): those
+        // started, and this one, do the work
     }
     work(0);
     for (int t = 0; t < started; ++t) pool[t].join();
