@@ -65,10 +65,10 @@ hipError_t ReadStaging::copy(const HostCopy* copies, int n, hipStream_t stream, 
     }
     const size_t chunks_all = (total + SLOT - 1) / SLOT;
     std::unique_lock<std::mutex> mine(busy_, std::defer_lock);
-    // The threads' start and the smaller transfers cost what they save up to 3 chunks (1.6 MB 119 us
-    // staged, 97 by hipMemcpy; 2.1 MB 125 and 127; 3.1 MB 164 and 190; 8.4 MB 395 and 500).  A
-    // second thread that reads the same context meanwhile has the runtime's copy too.
-    if (!staged || chunks_all < 4 || !mine.try_lock() || !reserve()) {
+    // Below 4 MiB the threads' start costs what they save (3.15 MB 190 us staged, 181 by hipMemcpy;
+    // 3.84 MB 210 and 214; 4.32 MB 222 and 247; 6.3 MB 303 and 354).  A second thread that reads the
+    // same context meanwhile has the runtime's copy too.
+    if (!staged || total < 4 * SLOT || !mine.try_lock() || !reserve()) {
         for (int i = 0; i < n; ++i) {
             if (!copies[i].bytes) continue;
             const hipError_t e = hipMemcpy(copies[i].dst, copies[i].src, copies[i].bytes, hipMemcpyDeviceToHost);

@@ -5,9 +5,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <atomic>
-#include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "readback.hpp"
@@ -16,6 +16,7 @@ static std::atomic<bool> no_memory{false};      // operator new refuses
 static std::atomic<int> staged{0}, plain{0};    // hipMemcpyAsync and hipMemcpy calls
 static std::atomic<int> fail_at{-1};            // the hipMemcpyAsync call that fails
 static std::atomic<bool> no_pinned{false};
+static std::atomic<int> second{0};              // a second reader: 1 expected, 2 done
 
 void* operator new(size_t n) {
     if (no_memory.load()) throw std::bad_alloc();
@@ -50,6 +51,7 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     if (staged++ == fail_at.load()) return hipErrorUnknown;
+    while (second.load() == 1) std::this_thread::yield();
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -63,10 +65,21 @@ int main(int argc, char** argv) {
     linon::ReadStaging staging;
     const size_t cut = bytes / 3;  // two copies, neither a whole number of chunks
     const linon::HostCopy copies[2] = {{dst.data(), src.data(), cut}, {dst.data() + cut, src.data() + cut, bytes - cut}};
-    no_memory = what == "no_memory";
     no_pinned = what == "no_pinned";
     fail_at = what == "fail" ? 3 : -1;
+    second = what == "second" ? 1 : 0;
+    std::thread reader;
+    std::vector<unsigned char> other(bytes, 0);
+    if (second == 1)
+        reader = std::thread([&] {  // while the first holds the slots
+            while (!staged.load()) std::this_thread::yield();
+            const linon::HostCopy copy{other.data(), src.data(), bytes};
+            if (staging.copy(&copy, 1, nullptr, 0) != hipSuccess || other != src) std::exit(4);
+            second = 2;
+        });
+    no_memory = what == "no_memory";
     const hipError_t e = staging.copy(copies, 2, nullptr, 0);
+    if (reader.joinable()) reader.join();
     no_memory = false;
     staging.release();
     std::printf("error %d equal %d staged %d plain %d\n", (int)e, (int)(src == dst), staged.load(), plain.load());

@@ -56,3 +56,22 @@ def test_read_back_from_two_threads():
         t.join()
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g, w)
+
+
+def test_two_threads_read_one_context():
+    """One of them through the staging, the other meanwhile by the runtime's copy, each as it comes."""
+    view = frame(1024, 700)
+    want = view.read_mapping()
+    got = [[], []]
+
+    def read(i):
+        for _ in range(5):
+            got[i].append(view.read_mapping())
+
+    threads = [threading.Thread(target=read, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g in got[0] + got[1]:
+        np.testing.assert_array_equal(g, want)

@@ -43,3 +43,15 @@ def test_a_failed_transfer_is_reported(driver):
 def test_no_pinned_memory(driver):
     r = driver("no_pinned")
     assert r["error"] == 0 and r["equal"] and (r["staged"], r["plain"]) == (0, 2)
+
+
+@pytest.mark.parametrize("size, staged", [((4 << 20) - 1, False), (4 << 20, True)])
+def test_copies_from_4_mib_are_staged(driver, size, staged):
+    r = driver("size", size)
+    assert r["error"] == 0 and r["equal"] and (r["staged"] > 0, r["plain"] > 0) == (staged, not staged)
+
+
+def test_a_second_reader_has_the_runtimes_copy(driver):
+    """Two threads read one context: the second does not wait for the first one's slots."""
+    r = driver("second")
+    assert r["error"] == 0 and r["equal"] and (r["staged"], r["plain"]) == (11, 1)
