@@ -233,8 +233,8 @@ linon_status linon_set_mesh(linon_context* ctx, const float* xyz, uint32_t num_v
                             const uint32_t* faces, uint32_t num_faces);
 linon_status linon_set_accel(linon_context* ctx, int accel, int grid_resolution);
 /* Where linon_set_mesh builds the grid: host threads or device kernels, which produce the same
- * arrays; AUTO builds on the device, and on the host where the device has no memory for that.
- * Rebuilds a mesh already set.
+ * arrays; AUTO builds on the device, and on the host grids of a few cells and where the device has
+ * no memory for the build.  Rebuilds a mesh already set.
  * (The reference has no acceleration structure: ray_color loops over all faces,
  * src/main_view.wgsl:177-220.) */
 typedef enum linon_grid_builder {

@@ -411,8 +411,8 @@ class MainView:
         self._check(self._lib.linon_set_math(self._h, math))
 
     def set_grid_builder(self, builder: int = GRID_BUILD_AUTO) -> None:
-        """Host threads or device kernels build the grid (same arrays); AUTO: device.
-        Rebuilds the current mesh."""
+        """Host threads or device kernels build the grid (same arrays); AUTO: device,
+        but for grids of a few cells.  Rebuilds the current mesh."""
         self._check(self._lib.linon_set_grid_builder(self._h, builder))
 
     def read_grid(self) -> dict:

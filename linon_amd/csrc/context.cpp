@@ -293,14 +293,18 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
         if (faces[i] >= nv) return fail(LINON_ERR_ARGUMENT, "set_mesh: face index out of range");
     int res = grid_res_req;
     if (res == 0) res = (nf <= 65536) ? 128 : 256;
-    // AUTO builds on the device at every size: 36 faces in 128^3 cells take 0.4 ms there and 27 ms
-    // on 16 host threads (the distance field alone is 2 M cells), 20,516 faces 0.75 and 30 ms,
-    // 1.3 M in 256^3 cells 19 ms and 1.2 s.  The host build is what is left where the device has
-    // no room for the build's scratch.
-    if (grid_builder != LINON_GRID_BUILD_HOST) {
-        GridGeom geo;
-        std::string e;
-        if (!grid_geometry(xyz, nv, faces, nf, res, geo, e)) return fail(LINON_ERR_ARGUMENT, "set_mesh: " + e);
+    GridGeom geo;
+    std::string e;
+    if (grid_builder != LINON_GRID_BUILD_HOST && !grid_geometry(xyz, nv, faces, nf, res, geo, e))
+        return fail(LINON_ERR_ARGUMENT, "set_mesh: " + e);
+    // AUTO builds on the device but for the tiniest grids: 36 faces in 128^3 cells take 0.4 ms there
+    // and 27 ms on 16 host threads (the distance field alone is 2 M cells), 20,516 faces 0.75 and 30
+    // ms, 1.3 M in 256^3 cells 18 ms and 1.2 s; 36 in 8^3 cells 0.19 and 0.10 ms.  The host build is
+    // also what is left where the device has no memory for the build.
+    const bool on_device =
+        grid_builder == LINON_GRID_BUILD_DEVICE ||
+        (grid_builder == LINON_GRID_BUILD_AUTO && (nf == 0 || !grid_is_tiny(geo, xyz, faces, nf)));
+    if (on_device) {
         // host copies: a later linon_set_accel may rebuild the grid (from them)
         const bool own = h_xyz.data() == xyz && h_faces.data() == faces;
         std::vector<float> new_xyz;
@@ -354,7 +358,6 @@ linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t*
                         "set_mesh: " + e);
     }
     GridBuild g;
-    std::string e;
     if (!build_grid(xyz, nv, faces, nf, res, g, e)) return fail(LINON_ERR_ARGUMENT, "set_mesh: " + e);
     std::vector<float> packed;
     pack_faces(xyz, faces, nf, packed);

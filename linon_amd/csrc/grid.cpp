@@ -102,6 +102,24 @@ bool grid_geometry(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_
     return true;
 }
 
+static void face_vertices(const float* xyz, const uint32_t* faces, size_t f, double v[3][3]) {
+    for (int j = 0; j < 3; ++j)
+        for (int k = 0; k < 3; ++k) v[j][k] = xyz[3 * (size_t)faces[3 * f + j] + k];
+}
+
+bool grid_is_tiny(const GridGeom& geo, const float* xyz, const uint32_t* faces, uint32_t nf) {
+    if ((size_t)geo.dim[0] * geo.dim[1] * geo.dim[2] > 2048) return false;
+    size_t tests = 0;
+    for (uint32_t f = 0; f < nf && tests <= 3072; ++f) {
+        double v[3][3];
+        face_vertices(xyz, faces, f, v);
+        int c0[3], c1[3];
+        face_cell_range(geo, v, c0, c1);
+        tests += (size_t)(c1[0] - c0[0] + 1) * (c1[1] - c0[1] + 1) * (c1[2] - c0[2] + 1);
+    }
+    return tests <= 3072;
+}
+
 bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf, int resolution,
                 GridBuild& g, std::string& err) {
     g = GridBuild();
@@ -124,8 +142,7 @@ bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t n
         std::vector<uint64_t>& out = pairs[tid];
         for (size_t f = b; f < e; ++f) {
             double v[3][3];
-            for (int j = 0; j < 3; ++j)
-                for (int k = 0; k < 3; ++k) v[j][k] = xyz[3 * (size_t)faces[3 * f + j] + k];
+            face_vertices(xyz, faces, f, v);
             int c0[3], c1[3];
             face_cell_range(geo, v, c0, c1);
             for (int z = c0[2]; z <= c1[2]; ++z)

@@ -9,6 +9,8 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+from linon_amd import scenes
+
 ROOT = Path(__file__).resolve().parent.parent
 CSRC = ROOT / "linon_amd" / "csrc"
 
@@ -55,3 +57,15 @@ def test_no_launch_has_too_many_lanes(lib):
         assert lib.stride_blocks(C.c_size_t(lanes)) * 256 < 2**32
     for lanes in (1, 16, 256, 257, 16 * 20516, (1 << 22) - 1):
         assert lanes <= lib.stride_blocks(C.c_size_t(lanes)) * 256 < lanes + 256
+
+
+def test_which_grids_the_host_builds(lib):
+    """Up to 2048 cells and 3072 overlap tests; a test for every cell of a face's range."""
+    box = scenes.cornell_box_centered()
+    for mesh, res, tiny in ((box, 4, 1), (box, 12, 1), (box, 16, 0), (box, 128, 0), (flat(1.0, 1.0), 45, 1),
+                            (flat(1.0, 1.0), 46, 0), (scenes.benchmark_scene(2), 8, 1),
+                            (scenes.benchmark_scene(2), 16, 0), (scenes.benchmark_scene(5), 128, 0)):
+        assert lib.grid_is_tiny(*arrays(*mesh)[2], res) == tiny, (len(mesh[1]), res)
+    v, f = flat(1.0, 1.0)  # three faces of 1024 cells each are the line
+    assert lib.grid_is_tiny(*arrays(v, np.tile(f, (3, 1)))[2], 32) == 1
+    assert lib.grid_is_tiny(*arrays(v, np.tile(f, (4, 1)))[2], 32) == 0
