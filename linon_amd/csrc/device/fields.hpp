@@ -122,7 +122,8 @@ using FieldLensRecip = FieldLensT<true>;
 // fewer instructions per step.  The temperature enters the step only through the refraction
 // indices, whose relative slope is at most 3.5e-3 per degree: an ulp of the sigmoid moves them
 // by about 1e-8, below the index ratio's own rounding.
-template <bool FaithfulRoot>
+// SideBranch: how refraction takes the side of the surface (refraction_impl).
+template <bool FaithfulRoot, bool SideBranch = false>
 struct FieldHotAirT {
     __device__ __forceinline__ static vec3 offset(vec3 q) { return q - vec3f(0.0f, -0.5f, 0.0f); }
     __device__ __forceinline__ static float distance(vec3 q) {
@@ -152,10 +153,10 @@ struct FieldHotAirT {
         return normalize(offset(p));
     }
     __device__ __forceinline__ vec3 operator()(vec3 p_prev, vec3 p, vec3, vec3 v, float) const {
-        return refraction_in_range(temperature(p_prev), temperature(p), v, normal(p));
+        return refraction_in_range<SideBranch>(temperature(p_prev), temperature(p), v, normal(p));
     }
     __device__ __forceinline__ vec3 first_stage(vec3 p, vec3, vec3 v, float) const {
-        return refraction_in_range_same(temperature(p), v, normal(p));
+        return refraction_in_range_same<SideBranch>(temperature(p), v, normal(p));
     }
 };
 using FieldHotAir = FieldHotAirT<false>;

@@ -389,12 +389,22 @@ __device__ __forceinline__ float mul_rounded(float a, float b) {  // a product t
 #pragma clang fp contract(off)
     return a * b;
 }
-template <bool InRange>
+// The side of the surface: n_ref = n where cosi < 0, -n elsewhere, and |cosi|.  SideBranch: by the
+// shader's branch.  Otherwise by the root's sign: rounding is symmetric in sign, so the factor of
+// n_ref and n_ref may both change sign together.  The results are the same but for the sign of an
+// exact zero; which is faster depends on the kernel (refraction_impl).
+template <bool InRange, bool SideBranch>
 __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_in, vec3 n) {
     auto quot = [](float a, float b) { return InRange ? div_in_range(a, b) : a / b; };
     float eta_in = quot(refraction_index_num(t_in), refraction_index_den(t_in));
     float eta_out = quot(refraction_index_num(t_out), refraction_index_den(t_out));
-    const float cosi = clamp(-1.0f, 1.0f, dot(v_in, n));
+    float cosi = clamp(-1.0f, 1.0f, dot(v_in, n));
+    if constexpr (SideBranch) {
+        if (cosi < 0.0f)
+            cosi = -cosi;
+        else
+            n = -n;
+    }
     float eta = quot(eta_in, eta_out);
     // k = RN(1 - e t), e = RN(eta eta), t = RN(1 - cosi cosi) in [0, 1] (the FMA form the
     // contracted expression 1 - eta * eta * (1 - cosi * cosi) compiles to).  k is never in
@@ -402,16 +412,16 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     // exponents of e and t add up to at least -2 and e t is a multiple of 2^-48, as is 1 - e t.
     // The root therefore needs no rescaling of tiny operands.
     const float k = __builtin_fmaf(-(eta * eta), __builtin_fmaf(-cosi, cosi, 1.0f), 1.0f);
-    // The shader's eta v_in + (eta |cosi| - sqrt(k)) n_ref, n_ref = n where cosi < 0 and -n
-    // elsewhere, with its contraction written out: fma(eta, v_i, RN(X n_ref_i)), X = fma(eta, |cosi|,
-    // -sqrt(k)) (the form the compiler picked for the expression).  Rounding is symmetric in sign,
-    // so X and n_ref may both change sign together: X n_ref = Y n with Y = fma(-eta, cosi, +-sqrt(k)),
-    // the root negated where cosi < 0.  One select instead of a branch over the side: its exec mask
-    // and moves took about 25 cycles a stage where a wave has its SIMD to itself (96x64 hot air's
-    // sample rays 5.3 -> 4.9 ms; 1080p hot air 13.55 -> 13.47 ms, plane mirage 13.55 -> 12.48).  With
+    // The shader's eta v_in + (eta |cosi| - sqrt(k)) n_ref with its contraction written out: fma(eta,
+    // v_i, RN(X n_ref_i)), X = fma(eta, |cosi|, -sqrt(k)) (the form the compiler picked for the
+    // expression); with n, X n_ref = Y n, Y = fma(-eta, cosi, +-sqrt(k)), the root negated where cosi
+    // < 0.  One select instead of a branch over the side: its exec mask and moves took about 25 cycles
+    // a stage where a wave has its SIMD to itself (a 96x64 frame of the spherical sigmoid mirage, all
+    // sample rays, 5.3 -> 4.9 ms; 1080p hot air 13.55 -> 13.47 ms, plane mirage 13.55 -> 12.48).  With
     // copysign(root, cosi) in place of the select, 1080p hot air takes 13.85.  NaN where k < 0.
     const float root = sqrt_rn_no_tiny(k);
-    const float Y = __builtin_fmaf(-eta, cosi, cosi < 0.0f ? -root : root);
+    const float Y = SideBranch ? __builtin_fmaf(eta, cosi, -root)
+                               : __builtin_fmaf(-eta, cosi, cosi < 0.0f ? -root : root);
     vec3 out = {__builtin_fmaf(eta, v_in.x, mul_rounded(Y, n.x)),
                 __builtin_fmaf(eta, v_in.y, mul_rounded(Y, n.y)),
                 __builtin_fmaf(eta, v_in.z, mul_rounded(Y, n.z))};
@@ -419,7 +429,7 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     // without it (nearly all) carry no reflection code, not even with an empty lane mask
     // (the empty asm keeps the compiler from turning the branch into selects)
     if (__any(k < 0.0f)) {
-        asm volatile("");
+        if constexpr (!SideBranch) asm volatile("");
         const vec3 r = reflect(v_in, n);  // = reflect(v_in, -n)
         const bool tir = k < 0.0f;
         out = {tir ? r.x : out.x, tir ? r.y : out.y, tir ? r.z : out.z};
@@ -427,12 +437,13 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     return out;
 }
 __device__ __forceinline__ vec3 refraction(float t_in, float t_out, vec3 v_in, vec3 n) {
-    return refraction_impl<false>(t_in, t_out, v_in, n);
+    return refraction_impl<false, false>(t_in, t_out, v_in, n);
 }
 // refraction() for temperatures in [-250, 1e4] deg C (the predefined fields': hot air's lie in
 // [20, 100], the mirages' in [15, 200]); bit for bit the same result.
+template <bool SideBranch = false>
 __device__ __forceinline__ vec3 refraction_in_range(float t_in, float t_out, vec3 v_in, vec3 n) {
-    return refraction_impl<true>(t_in, t_out, v_in, n);
+    return refraction_impl<true, SideBranch>(t_in, t_out, v_in, n);
 }
 // refraction_in_range(t, t, v_in, n): one temperature on both sides, as in the first RK4 stage
 // of a field that compares T(p_prev) with T(p).  The index ratio n(t) / n(t) is then exactly 1
@@ -444,18 +455,26 @@ __device__ __forceinline__ vec3 refraction_in_range(float t_in, float t_out, vec
 // NaN t gives NaN in every component, as its NaN ratio does there (cosi - (t - t) is cosi for
 // a finite t).  The WGSL-accuracy build divides approximately, where n(t) / n(t) need not be
 // 1, and keeps the general form.
+template <bool SideBranch = false>
 __device__ __forceinline__ vec3 refraction_in_range_same(float t, vec3 v_in, vec3 n) {
 #ifdef LINON_FAST_MATH
-    return refraction_impl<true>(t, t, v_in, n);
+    return refraction_impl<true, SideBranch>(t, t, v_in, n);
 #else
-    const float cosi = clamp(-1.0f, 1.0f, dot(v_in, n)) - (t - t);
+    float cosi = clamp(-1.0f, 1.0f, dot(v_in, n)) - (t - t);
+    if constexpr (SideBranch) {
+        if (cosi < 0.0f)
+            cosi = -cosi;
+        else
+            n = -n;
+    }
     // 1 - t with t = RN(1 - cosi cosi) in [0, 1]: zero, or at least 2^-24 (t >= 1/2 is a
     // multiple of 2^-24) -- no tiny operand for the root; never negative, so never the total
     // internal reflection of the general form (a NaN t gives NaN there as here)
     const float k = 1.0f - __builtin_fmaf(-cosi, cosi, 1.0f);
     // (the sign here by copysign, of cosi + 0 since -0 is not < 0: 1080p hot air takes 13.9 ms with a
     // select in this stage too, 13.5 with it in the general form alone)
-    const float y = __builtin_copysignf(sqrt_rn_no_tiny(k), cosi + 0.0f) - cosi;
+    const float y = SideBranch ? cosi - sqrt_rn_no_tiny(k)
+                               : __builtin_copysignf(sqrt_rn_no_tiny(k), cosi + 0.0f) - cosi;
     auto axpy = [](float a, float b, float c) {
 #pragma clang fp contract(off)
         return a * b + c;
