@@ -10,7 +10,8 @@ namespace lw {
 
 // A functor may also define first_stage(p, v0, v, t) = (*this)(p, p, v0, v, t), bit for bit,
 // with less work; the integrators call it for the first RK4 stage, where p_prev == p.
-template <bool Spherical, bool Sigmoid>
+// SideBranch, here and in hot air: how refraction takes the side of the surface (refraction_impl).
+template <bool Spherical, bool Sigmoid, bool SideBranch = false>
 struct FieldMirage {  // src/functions.rs:36-96
     // distance from the hot source: the sphere's centre or the plane
     __device__ __forceinline__ static float distance_to_source(vec3 q) {
@@ -35,11 +36,11 @@ struct FieldMirage {  // src/functions.rs:36-96
         return part * t_env + (1.0f - part) * t_src;
     }
     __device__ __forceinline__ vec3 operator()(vec3 p_prev, vec3 p, vec3, vec3 v, float) const {
-        return refraction_in_range(temperature(distance_to_source(p_prev)), temperature(distance_to_source(p)), v,
-                                   normal_at(p));
+        return refraction_in_range<SideBranch>(temperature(distance_to_source(p_prev)),
+                                               temperature(distance_to_source(p)), v, normal_at(p));
     }
     __device__ __forceinline__ vec3 first_stage(vec3 p, vec3, vec3 v, float) const {
-        return refraction_in_range_same(temperature(distance_to_source(p)), v, normal_at(p));
+        return refraction_in_range_same<SideBranch>(temperature(distance_to_source(p)), v, normal_at(p));
     }
 };
 using FieldMirageSpherical = FieldMirage<true, false>;
@@ -122,7 +123,6 @@ using FieldLensRecip = FieldLensT<true>;
 // fewer instructions per step.  The temperature enters the step only through the refraction
 // indices, whose relative slope is at most 3.5e-3 per degree: an ulp of the sigmoid moves them
 // by about 1e-8, below the index ratio's own rounding.
-// SideBranch: how refraction takes the side of the surface (refraction_impl).
 template <bool FaithfulRoot, bool SideBranch = false>
 struct FieldHotAirT {
     __device__ __forceinline__ static vec3 offset(vec3 q) { return q - vec3f(0.0f, -0.5f, 0.0f); }

@@ -506,6 +506,12 @@ __device__ __forceinline__ bool ray_finished(const RayState& r, const StepParams
 // Stop: a predicate on the ray after each step; when it holds the loop returns early, with
 // ray_finished's verdict (the approach leg of a surrogate frame stops at the sphere).
 enum : int { LK_STEP_ANY = 0, LK_STEP_FIXED_REFERENCE = 1, LK_STEP_FIXED_ESCAPE = 2 };
+// The functor a loop evaluates for field F: one with the same results, where another form of it is
+// faster there (loop_fields.hpp).
+template <class F, bool WOne, int Fixed>
+struct LoopField {
+    using type = F;
+};
 struct NeverStop {
     static constexpr bool EACH_STEP = false;
     __device__ __forceinline__ bool operator()(const vec3&) const { return false; }
@@ -514,7 +520,7 @@ template <class F, bool WOne, int Fixed, class Stop = NeverStop>
 __device__ __forceinline__ bool ray_advance_impl(RayState& r, const StepParams& I, const SceneParams& S,
                                                  const float4* lds, int budget, QueryStats& st,
                                                  Stop stop = Stop{}) {
-    const F field{};
+    const typename LoopField<F, WOne, Fixed>::type field{};
     const bool adaptive = Fixed == LK_STEP_ANY ? I.adaptive != 0 : false;
     const bool escape = Fixed == LK_STEP_ANY ? (I.mode == LINON_MODE_ESCAPE) : Fixed == LK_STEP_FIXED_ESCAPE;
     const bool brute = (S.accel == LINON_ACCEL_BRUTE_K);

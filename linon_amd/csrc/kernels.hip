@@ -7,6 +7,7 @@
 
 #include "device/batch.hpp"
 #include "device/fields.hpp"
+#include "device/loop_fields.hpp"
 #include "device/raycast.hpp"
 #include "kernels.hpp"
 
@@ -17,22 +18,9 @@ __global__ void __launch_bounds__(64) LK_RAYCAST_OCCUPANCY raycast_kernel(Raycas
     lk::raycast_body<F>(P);
 }
 
-// The batch's functor of a field: in hot air's default variant refraction keeps the branch over the
-// side of the surface.  24 of the batch's views, all of one field, twelve runs of each in turn: that variant
-// 103.5 ms with the branch and 106.1 without; hot air IEEE 140.5 and 138.1, WGSL accuracy 131.2 and
-// 126.6; the mirages 103.4 and 96.7 (plane), 126.5 and 120.9 (plane sigmoid), 117.9 and 114.9
-// (spherical), 145.5 and 144.0 (spherical sigmoid).
-template <class F>
-struct BatchField {
-    using type = F;
-};
-template <>
-struct BatchField<lw::FieldHotAirFaithfulRoot> {
-    using type = lw::FieldHotAirT<true, true>;
-};
 template <class F>
 __global__ void __launch_bounds__(256) LK_BATCH_OCCUPANCY batch_kernel(BatchParams B) {
-    lk::batch_body<typename BatchField<F>::type>(B);
+    lk::batch_body<F>(B);
 }
 
 __global__ void __launch_bounds__(256) overlay_kernel(OverlayParams P) { lk::overlay_body(P); }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device/fields.hpp"
+#include "device/loop_fields.hpp"
 #include "device/gemm_nt.hpp"
 #include "device/gemm_tn.hpp"
 #include "device/mlp.hpp"
