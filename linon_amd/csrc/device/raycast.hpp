@@ -745,6 +745,11 @@ __device__ __forceinline__ void raycast_body(const RaycastParams& P) {
     const int lane = threadIdx.x;
     if (P.sample_block) {
         if (b == 0) {
+            // 48 bytes that put the pixels' step loops behind the sample rays' code back where they lay
+            // before that code got shorter: the fetch of a loop's instructions depends on its place
+            // (1365x767 swirl at h = 0.005 2.61 ms then, 2.66 without the bytes, 2.58 with them; 1080p
+            // 4.76, 4.84, 4.70; hot air 7.25, 7.19, 7.15; the other fields' loops change by less than 1%)
+            asm volatile(".rept 12\n\ts_nop 0\n\t.endr");
             // one wave for the 8 rays: with a block each, hence an XCD each, the slowest of the 8
             // took 10-15% longer than the one
             if (lane < 8 && P.ray_samples && P.samples_per_ray > 0) sample_rays<F>(P, cam, lane);
