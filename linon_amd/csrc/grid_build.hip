@@ -78,11 +78,15 @@ struct Reference {
 // projections of the three vertices on each of the 13 axes, widened by the box's half extent.  A
 // cell is then settled by the projection of its centre, about 70 double-precision operations
 // where face_in_cell takes 350, unless some axis comes within a slack of its threshold, which
-// covers the rounding of both computations; those cells (about one in 10^11) take face_in_cell
-// itself.  With |vertices|, |centres| <= S both projections onto an edge axis are off by less than
-// 2^-46 S^2, onto the normal by less than 2^-42 S^3, and onto a box axis by 2^-50 S; the slacks are
-// 8 times that and more.  An axis that is exactly zero (an edge along it: the difference of equal
-// coordinates is zero in both computations) separates nothing and has infinite thresholds.
+// covers the rounding of both computations; those cells take face_in_cell itself.  With |vertices|,
+// |centres| <= S both projections onto an edge axis are off by less than 2^-46 S^2, onto the normal
+// by less than 2^-42 S^3, and onto a box axis by 2^-50 S; the slacks are 8 times that and more.  For
+// a mesh about the origin about one cell in 10^11 comes so close.  They grow with the distance from
+// the origin, not the mesh's size, and a face without area has a normal of zero, which always does:
+// 327,716 faces in 256^3 cells take 6.4 ms about the origin, 9.6 at 100 units from it and 9.7 at
+// 1000, 7.1 without area (by face_in_cell alone, one lane a face, 14.7, 20.5, 14.7 and 13.8).  An
+// axis that is exactly zero (an edge along it: the difference of equal coordinates is zero in both
+// computations) separates nothing and has infinite thresholds.
 struct FaceTest {
     double e[3][3];            // edges
     double lo[9], hi[9];       // thresholds of the edge axes (3 j + i: edge j x unit vector i)

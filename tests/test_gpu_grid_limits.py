@@ -140,3 +140,21 @@ def test_a_refused_mesh_leaves_the_present_one(builder):
         view.set_accel(L.ACCEL_GRID, 64)   # rebuilt from the context's own copy of the mesh
         view.render()
         assert (view.read_hit_faces() >= 0).any()
+
+
+@pytest.mark.parametrize("offset", [0.0, 100.0, 1000.0, 1e6])
+@pytest.mark.parametrize("area", [True, False])
+def test_faces_far_from_the_origin_and_without_area(offset, area):
+    """The short overlap test leaves the cells near an axis's threshold to the full one: more of them the
+    further the mesh is from the origin, and every cell of a face that is a line or a point."""
+    v, f = scenes.benchmark_scene(level=3)
+    f = f.copy()
+    if not area:
+        f[::2, 2] = f[::2, 1]
+        f[::8] = f[::8, :1]
+    print(f"[case] grid build {offset} from the origin, area {area}", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_accel(L.ACCEL_GRID, 64)
+        view.update_model((v + np.float32(offset)).astype(np.float32), f)
+        d = same_grids(view)
+    assert len(d["cell_faces"]) > len(f)
