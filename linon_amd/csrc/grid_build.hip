@@ -156,7 +156,7 @@ struct FaceTest {
 };
 
 // Lists the faces that face_overlap_kernel leaves alone: mid ones from the front of big[nf], huge
-// ones from its back; nbig[2] counts them.  One atomic per class and block of 1024 faces: they all
+// ones from its back; nbig[0] and nbig[1] count them.  One atomic per class and block of 1024 faces: they all
 // go to two addresses, about 9 ns each.
 __global__ void __launch_bounds__(1024) classify_kernel(GridGeom g, const float* xyz, const uint32_t* faces,
                                                         uint32_t nf, unsigned* big, unsigned* nbig) {
@@ -335,15 +335,90 @@ __global__ void __launch_bounds__(256) list_kernel(const Reference* refs, size_t
 // Each reference to its rank in its cell: the ascending order of the face ids (distinct in a
 // cell).  A lane compares against its cell's whole list, so a list of L faces takes L^2
 // comparisons side by side, where an insertion sort by one lane takes as many in a chain (0.9 ms
-// for 1.3 M faces in 256^3 cells).
+// for 1.3 M faces in 256^3 cells).  Lists beyond kLongList are left to long_list_kernel; their
+// cells go to long_cells.
+constexpr unsigned kLongList = 256;
 __global__ void __launch_bounds__(256) rank_kernel(const Reference* refs, size_t n, const unsigned* cell_start,
-                                                   const unsigned* list, unsigned* cell_faces) {
+                                                   const unsigned* list, unsigned* cell_faces, unsigned* long_cells,
+                                                   unsigned* nlong) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const Reference r = refs[i];
         const unsigned b = cell_start[r.cell], e = cell_start[r.cell + 1];
+        if (e - b > kLongList) {
+            if (r.slot == 0) long_cells[atomicAdd(nlong, 1u)] = r.cell;
+            continue;
+        }
         unsigned rank = 0;
         for (unsigned j = b; j < e; ++j) rank += list[j] < r.face ? 1u : 0u;
         cell_faces[(size_t)b + rank] = r.face;
+    }
+}
+
+// Sorts each long list, a block of 1024 a list: radix passes of 8 bits, lowest first, between `list`
+// and `cell_faces`, an odd number of them so that the last ends in cell_faces.  Ranked like the short
+// ones, L faces in the same C cells take C L^2 comparisons: 4,000 full-size walls in 128^3 cells
+// RANK_MS, and 20,000 as long as the host RANK20; so they take SORT_MS.
+__global__ void __launch_bounds__(1024) long_list_kernel(const unsigned* cell_start, unsigned* list,
+                                                         unsigned* cell_faces, const unsigned* long_cells,
+                                                         const unsigned* nlong, int passes) {
+    __shared__ unsigned at[256], wave_at[16][256];
+    const unsigned t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    for (unsigned i = blockIdx.x; i < *nlong; i += gridDim.x) {
+        const unsigned b = cell_start[long_cells[i]], n = cell_start[long_cells[i] + 1] - b;
+        for (int p = 0; p < passes; ++p) {
+            const unsigned* in = (p & 1 ? cell_faces : list) + b;
+            unsigned* out = (p & 1 ? list : cell_faces) + b;
+            const int shift = 8 * p;
+            auto digit = [&](unsigned x) { return shift < 32 ? (x >> shift) & 255u : 0u; };
+            if (t < 256) at[t] = 0;
+            __syncthreads();
+            for (unsigned j = t; j < n; j += 1024) atomicAdd(&at[digit(in[j])], 1u);
+            __syncthreads();
+            // where each digit's faces begin: one wave, four digits a lane
+            if (t < 64) {
+                unsigned c[4], sum = 0;
+                for (int k = 0; k < 4; ++k) {
+                    c[k] = at[4 * t + k];
+                    sum += c[k];
+                }
+                unsigned upto = sum;
+                for (unsigned off = 1; off < 64; off <<= 1) {
+                    const unsigned x = __shfl_up(upto, off, 64);
+                    if (lane >= off) upto += x;
+                }
+                unsigned begin = upto - sum;
+                for (int k = 0; k < 4; ++k) {
+                    at[4 * t + k] = begin;
+                    begin += c[k];
+                }
+            }
+            for (unsigned j0 = 0; j0 < n; j0 += 1024) {
+                for (unsigned k = t; k < 16 * 256; k += 1024) wave_at[k >> 8][k & 255] = 0;
+                __syncthreads();
+                const bool have = j0 + t < n;
+                const unsigned x = have ? in[j0 + t] : 0u, d = digit(x);
+                unsigned long long same = __ballot(have);  // the wave's lanes of this digit
+                for (int bit = 0; bit < 8; ++bit) {
+                    const unsigned long long set = __ballot(d >> bit & 1u);
+                    same &= d >> bit & 1u ? set : ~set;
+                }
+                const unsigned before = (unsigned)__popcll(same & ((1ull << lane) - 1ull));
+                if (have && before == 0) wave_at[wave][d] = (unsigned)__popcll(same);
+                __syncthreads();
+                if (t < 256) {
+                    unsigned o = at[t];
+                    for (int w = 0; w < 16; ++w) {
+                        const unsigned k = wave_at[w][t];
+                        wave_at[w][t] = o;
+                        o += k;
+                    }
+                    at[t] = o;
+                }
+                __syncthreads();
+                if (have) out[wave_at[wave][d] + before] = x;
+                __syncthreads();  // before the counts are cleared, and before the next pass reads `out`
+            }
+        }
     }
 }
 
@@ -551,7 +626,7 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
     const int i_count = A.add<unsigned>(nf), i_first = A.add<unsigned>(nf), i_big = A.add<unsigned>(nf);
     const int i_cursor = A.add<unsigned>(nf), i_cells = A.add<unsigned>(nc);
     const int i_local = A.add<unsigned long long>(longest), i_bsum = A.add<unsigned long long>(max_blocks);
-    const int i_total = A.add<unsigned long long>(1), i_nbig = A.add<unsigned>(2), i_tmp = A.add<unsigned char>(nc);
+    const int i_total = A.add<unsigned long long>(1), i_nbig = A.add<unsigned>(3), i_tmp = A.add<unsigned char>(nc);
     GridResult result = GridResult::BUILT;
     auto check = [&](hipError_t e, const char* what) {
         if (e == hipSuccess) return true;
@@ -594,7 +669,7 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
                 return false;
             if (!check(hipMemcpyAsync(d_faces, h_faces, 3 * (size_t)nf * 4, hipMemcpyHostToDevice, s), "upload"))
                 return false;
-            hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, d_nbig, (size_t)2, 0u);
+            hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, s, d_nbig, (size_t)3, 0u);
             hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nf, 256)), dim3(256), 0, s, d_cursor, (size_t)nf, 0u);
             hipLaunchKernelGGL(classify_kernel, dim3(blocks_for(nf, 1024)), dim3(1024), 0, s, g, d_xyz, d_faces, nf,
                                d_big, d_nbig);
@@ -618,12 +693,13 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
             }
         }
         const int i_refs = R.add<Reference>((size_t)total), i_list = R.add<unsigned>((size_t)total);
+        const int i_long = R.add<unsigned>((size_t)total / kLongList);
         if (!check(alloc(&out.cell_faces, std::max<size_t>(1, (size_t)total) * 4), "alloc")) return false;
         out.refs = (size_t)total;
         if (total) {
             if (!check(R.allocate(alloc), "alloc")) return false;
             Reference* d_refs = R.get<Reference>(i_refs);
-            unsigned* d_list = R.get<unsigned>(i_list);
+            unsigned *d_list = R.get<unsigned>(i_list), *d_long = R.get<unsigned>(i_long);
             hipLaunchKernelGGL(face_place_kernel, dim3(face_blocks), dim3(256), 0, s, g, d_xyz, d_faces, nf,
                                (const unsigned short*)d_masks, (const unsigned*)d_first, d_cells, d_refs);
             big_overlap_kernel<false, true><<<mid_grid, 256, 0, s>>>(g, d_xyz, d_faces, nf, d_big, d_nbig, nullptr,
@@ -637,7 +713,14 @@ GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv,
                                (unsigned)total);
             hipLaunchKernelGGL(rank_kernel, dim3(stride_blocks((size_t)total)), dim3(256), 0, s,
                                (const Reference*)d_refs, (size_t)total, (const unsigned*)out.cell_start,
-                               (const unsigned*)d_list, out.cell_faces);
+                               (const unsigned*)d_list, out.cell_faces, d_long, d_nbig + 2);
+            if (nf > kLongList) {  // (a shorter mesh has no such list)
+                int passes = 1;
+                while (passes < 4 && (nf - 1) >> (8 * passes)) ++passes;
+                hipLaunchKernelGGL(long_list_kernel, dim3(512), dim3(1024), 0, s, (const unsigned*)out.cell_start,
+                                   d_list, out.cell_faces, (const unsigned*)d_long, (const unsigned*)(d_nbig + 2),
+                                   passes | 1);
+            }
         } else {
             hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(nc + 1, 256)), dim3(256), 0, s, out.cell_start, nc + 1,
                                0u);

@@ -158,3 +158,21 @@ def test_faces_far_from_the_origin_and_without_area(offset, area):
         view.update_model((v + np.float32(offset)).astype(np.float32), f)
         d = same_grids(view)
     assert len(d["cell_faces"]) > len(f)
+
+
+# lists about the line between the ranks and the sort (256), with one, two and three bytes of face id,
+# and last chunks of one
+@pytest.mark.parametrize("n", [250, 256, 257, 262, 300, 1025, 2049, 3073, 70001])
+def test_long_lists(n):
+    """n faces in a few cells about the centre, some of them reaching far, and two that span the grid."""
+    rng = np.random.default_rng(n)
+    v = rng.normal(size=(n, 3, 3)) * 1e-3
+    v[::97] *= 100.0
+    v = np.concatenate([v.reshape(-1, 3), [[-1, -1, -1], [1, 1, 1], [1, 1.01, 1], [-1, 0, 0], [1, 0, 0], [0, 1, 0]]])
+    f = rng.permutation(np.arange(3 * n + 6, dtype=np.uint32).reshape(-1, 3))
+    print(f"[case] {n} faces in a few cells", flush=True)
+    with L.MainView(16, 16) as view:
+        view.set_accel(L.ACCEL_GRID, 33)
+        view.update_model(v.astype(np.float32), f)
+        d = same_grids(view)
+    assert np.diff(d["cell_start"]).max() > 0.98 * n
