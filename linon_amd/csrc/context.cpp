@@ -289,6 +289,14 @@ linon_status Context::read_all(const HostCopy* copies, int n) {
 }
 
 linon_status Context::upload_mesh(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf) {
+    try {
+        return build_mesh(xyz, nv, faces, nf);
+    } catch (const std::bad_alloc&) {  // of the host: nothing may leave a C entry
+        return fail(LINON_ERR_HIP, "set_mesh: out of host memory");
+    }
+}
+
+linon_status Context::build_mesh(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf) {
     for (size_t i = 0; i < 3 * (size_t)nf; ++i)
         if (faces[i] >= nv) return fail(LINON_ERR_ARGUMENT, "set_mesh: face index out of range");
     int res = grid_res_req;

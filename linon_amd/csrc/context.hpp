@@ -159,6 +159,7 @@ struct Context {
     void free_mesh();
     void release_jit();
     linon_status upload_mesh(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf);
+    linon_status build_mesh(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf);
     bool srgb_output = false;  // overlay_web epilogue
     int num_cus = 0;
 

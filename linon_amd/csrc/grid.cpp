@@ -6,6 +6,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <exception>
+#include <mutex>
 #include <thread>
 
 namespace linon {
@@ -25,22 +27,41 @@ void pack_faces(const float* xyz, const uint32_t* faces, uint32_t nf, std::vecto
     }
 }
 
+// fn(begin, end, thread) over [0, n) in `nt` pieces.  What a piece throws (std::bad_alloc) is thrown
+// again here once every thread has ended; a piece without a thread to be had runs on this one.
 template <class Fn>
-static void parallel_for(size_t n, Fn fn) {
-    unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+static void parallel_for(size_t n, unsigned nt, Fn fn) {
     if (n < 4096 || nt == 1) {
         fn(0, n, 0u);
         return;
     }
     std::vector<std::thread> th;
-    size_t chunk = (n + nt - 1) / nt;
+    std::exception_ptr thrown;
+    std::mutex guard;
+    const size_t chunk = (n + nt - 1) / nt;
+    auto piece = [&](size_t b, size_t e, unsigned t) {
+        try {
+            fn(b, e, t);
+        } catch (...) {
+            const std::lock_guard<std::mutex> lock(guard);
+            thrown = std::current_exception();
+        }
+    };
+    th.reserve(nt);
     for (unsigned t = 0; t < nt; ++t) {
-        size_t b = t * chunk, e = std::min(n, b + chunk);
+        const size_t b = t * chunk, e = std::min(n, b + chunk);
         if (b >= e) break;
-        th.emplace_back(fn, b, e, t);
+        try {
+            th.emplace_back(piece, b, e, t);
+        } catch (...) {
+            piece(b, e, t);
+        }
     }
     for (auto& x : th) x.join();
+    if (thrown) std::rethrow_exception(thrown);
 }
+
+static unsigned build_threads() { return std::max(1u, std::min(16u, std::thread::hardware_concurrency())); }
 
 // min over j of max(|i - j|, g[j]) along one line of n samples with stride s, searched
 // outwards from i and stopped once the offset alone reaches the best value found.
@@ -136,9 +157,9 @@ bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t n
     const size_t nc = g.ncells();
 
     // (cell, face) pairs, one vector per thread over ascending face ranges
-    unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    const unsigned nt = build_threads();
     std::vector<std::vector<uint64_t>> pairs(nt);
-    auto emit = [&](size_t b, size_t e, unsigned tid) {
+    parallel_for(nf, nt, [&](size_t b, size_t e, unsigned tid) {
         std::vector<uint64_t>& out = pairs[tid];
         for (size_t f = b; f < e; ++f) {
             double v[3][3];
@@ -153,19 +174,7 @@ bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t n
                             out.push_back((cell << 32) | (uint64_t)f);
                         }
         }
-    };
-    if (nf < 4096 || nt == 1) {
-        emit(0, nf, 0);
-    } else {
-        std::vector<std::thread> th;
-        size_t chunk = (nf + nt - 1) / nt;
-        for (unsigned t = 0; t < nt; ++t) {
-            size_t b = t * chunk, e = std::min<size_t>(nf, b + chunk);
-            if (b >= e) break;
-            th.emplace_back(emit, b, e, t);
-        }
-        for (auto& x : th) x.join();
-    }
+    });
     // counting sort by cell, stable in (thread, face) order = ascending faces per cell
     g.cell_start.assign(nc + 1, 0u);
     size_t total = 0;
@@ -188,7 +197,7 @@ bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t n
 
     // Chebyshev distance (in cells, capped at 255) from every cell to the nearest occupied one
     std::vector<uint8_t> a(nc), b(nc);
-    parallel_for((size_t)ny * nz, [&](size_t lb, size_t le, unsigned) {
+    parallel_for((size_t)ny * nz, nt, [&](size_t lb, size_t le, unsigned) {
         for (size_t line = lb; line < le; ++line) {
             size_t base = line * nx;
             int d = 255;
@@ -204,14 +213,14 @@ bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t n
             }
         }
     });
-    parallel_for((size_t)nz * nx, [&](size_t lb, size_t le, unsigned) {
+    parallel_for((size_t)nz * nx, nt, [&](size_t lb, size_t le, unsigned) {
         for (size_t line = lb; line < le; ++line) {
             size_t z = line / nx, x = line % nx;
             size_t base = z * (size_t)nx * ny + x;
             minmax_line(a.data() + base, b.data() + base, ny, (size_t)nx);
         }
     });
-    parallel_for((size_t)ny * nx, [&](size_t lb, size_t le, unsigned) {
+    parallel_for((size_t)ny * nx, nt, [&](size_t lb, size_t le, unsigned) {
         for (size_t line = lb; line < le; ++line) {
             minmax_line(b.data() + line, a.data() + line, nz, (size_t)nx * ny);
         }

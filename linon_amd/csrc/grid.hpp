@@ -35,7 +35,8 @@ bool grid_geometry(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_
 // cells empty), 225 at 4096 and 4550, 505 at 4096 of each.
 bool grid_is_tiny(const GridGeom& geo, const float* xyz, const uint32_t* faces, uint32_t nf);
 
-// Builds the grid on the host (threads).  Returns false and sets `err` for invalid input.
+// Builds the grid on the host (threads).  Returns false and sets `err` for invalid input; throws
+// std::bad_alloc, from the calling thread alone, where memory ends.
 bool build_grid(const float* xyz, uint32_t nv, const uint32_t* faces, uint32_t nf, int resolution,
                 GridBuild& g, std::string& err);
 

@@ -69,3 +69,18 @@ def test_which_grids_the_host_builds(lib):
     v, f = flat(1.0, 1.0)  # three faces of 1024 cells each are the line
     assert lib.grid_is_tiny(*arrays(v, np.tile(f, (3, 1)))[2], 32) == 1
     assert lib.grid_is_tiny(*arrays(v, np.tile(f, (4, 1)))[2], 32) == 0
+
+
+def test_no_memory_for_the_host_build(tmp_path):
+    """Wherever in the host build memory ends, in a thread of it too, the caller gets std::bad_alloc (and
+    the C entry an error); nothing is left running."""
+    exe = tmp_path / "grid_memory_driver"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{CSRC}",
+                    str(ROOT / "tests" / "host" / "grid_memory_driver.cpp"), str(CSRC / "grid.cpp"), "-pthread",
+                    "-o", str(exe)], check=True)
+    said = []
+    for k in range(4, 31):
+        r = subprocess.run([str(exe), str(1 << k)], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, (k, r.returncode, r.stderr[-300:])
+        said.append(r.stdout.strip())
+    assert said[0] == "no memory" and said[-1] == "built"
