@@ -640,8 +640,10 @@ __device__ __forceinline__ bool ray_advance_impl(RayState& r, const StepParams& 
 // step cap make one condition, so that a step has one branch and one change of the lane mask (the
 // general loop has fifteen blocks and 55 scalar instructions a step without a mesh too, here 17).
 // What bounds it: VALU issue, sines quarter rate; a flow map of few rays, the chain of a step.
-// 50,001 hot-air rays 770 -> 680 us, the approach and re-judging legs of a 1080p warp frame 1.20 ->
-// 1.14 ms and 184 -> 157 us.
+// 50,001 rays, the general loop and this one: hot air 757 -> 649 us, swirl 273 -> 205, warp 297 ->
+// 229; 400,000: 2718 -> 2627, 976 -> 924, 748 -> 730.  (With the outward test at every step 400,000
+// rays took 2733, 1052 and 811: more instructions than the general loop, which branches past it.)
+// The approach leg of a 1080p warp frame 1.36 -> 1.01 ms.
 template <class F, bool WOne, class Stop = NeverStop>
 __device__ __forceinline__ bool ray_advance_free(RayState& r, const StepParams& I, Stop stop = Stop{}) {
     const F field{};
@@ -668,8 +670,13 @@ __device__ __forceinline__ bool ray_advance_free(RayState& r, const StepParams& 
         step = rn::mul(r.d, h);
         q = rn::add(p, step);
         r.t = rn::add(r.t, h);
-        // (no && or ||: each would be a branch)
-        out = int(rn::dot(q, q) > I.escape_r2) & int(rn::dot(q, r.d) > 0.0f);
+        // (no && or ||: each would be a branch over lanes; the wave's branch leaves out the outward test
+        // of the steps, nearly all, in which no lane is beyond the sphere)
+        out = rn::dot(q, q) > I.escape_r2;
+        if (__any(out)) {
+            asm volatile("");
+            out = int(out) & int(rn::dot(q, r.d) > 0.0f);
+        }
         last = r.iters >= I.max_steps;
         return int(out) | int(last) | int(stop(q));
     };

@@ -408,10 +408,10 @@ static const void* approach_for(int field) {
 static const void* flowmap_for(int field) {
     switch (field) { LS_LENS_CASES(flowmap_kernel) LS_FIELD_CASES(flowmap_kernel) }
 }
-// Fixed steps in the loop without a mesh: 262,144 rays with their copies hot air 2.63 -> 2.33 ms, warp
-// 1.35 -> 1.25, mirage 3.72 -> 3.41, and 3,000 rays 10-30% less.  Not the lens, whose step is mostly
-// its field's own branches: 844,000 rays take 9.12 ms so and 8.97 in the general loop, 3,000 rays
-// 1.03-1.20 and 1.16 ms a call.
+// Fixed steps in the loop without a mesh: faster from one ray to 400,000 (ray_advance_free's
+// figures).  Not the lens, whose step is mostly its field's own branches: with the outward test at
+// every step 844,000 rays took 9.12 ms so and 8.97 in the general loop, 3,000 rays 1.03-1.20 and
+// 1.16 ms a call.
 static const void* flowmap_free_for(int field) {
     switch (field) { LS_FIELD_CASES(flowmap_free_kernel) }
 }
