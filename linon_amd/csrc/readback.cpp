@@ -58,17 +58,16 @@ bool pageable(const void* p) {
 
 hipError_t ReadStaging::copy(const HostCopy* copies, int n, hipStream_t stream, int device) {
     size_t total = 0;
-    bool staged = true;
-    for (int i = 0; i < n; ++i) {
-        total += copies[i].bytes;
-        staged = staged && (copies[i].bytes == 0 || pageable(copies[i].dst));
-    }
+    for (int i = 0; i < n; ++i) total += copies[i].bytes;
     const size_t chunks_all = (total + SLOT - 1) / SLOT;
     std::unique_lock<std::mutex> mine(busy_, std::defer_lock);
     // Below 4 MiB the threads' start costs what they save (3.15 MB 190 us staged, 181 by hipMemcpy;
-    // 3.84 MB 210 and 214; 4.32 MB 222 and 247; 6.3 MB 303 and 354).  A second thread that reads the
-    // same context meanwhile has the runtime's copy too.
-    if (!staged || total < 4 * SLOT || !mine.try_lock() || !reserve()) {
+    // 3.84 MB 210 and 214; 4.32 MB 222 and 247; 6.3 MB 303 and 354), and the question what memory the
+    // destination is up to 4% of a small read.  A second thread that reads the same context meanwhile
+    // has the runtime's copy too.
+    bool staged = total >= 4 * SLOT;
+    for (int i = 0; staged && i < n; ++i) staged = copies[i].bytes == 0 || pageable(copies[i].dst);
+    if (!staged || !mine.try_lock() || !reserve()) {
         for (int i = 0; i < n; ++i) {
             if (!copies[i].bytes) continue;
             const hipError_t e = hipMemcpy(copies[i].dst, copies[i].src, copies[i].bytes, hipMemcpyDeviceToHost);
