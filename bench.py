@@ -323,7 +323,7 @@ def main() -> int:
     # the kernel each field runs under the default math choice, as rocprofv3 names it
     kname = {"swirl": "linon_wgslmath::raycast_kernel<lw::FieldSwirl>",
              "lens": "linon::raycast_kernel<lw::FieldLensT<true> >",
-             "hot_air": "linon::raycast_kernel<lw::FieldHotAirT<true> >",
+             "hot_air": "linon::raycast_kernel<lw::FieldHotAirT<true, false> >",
              "warp": "linon_wgslmath::raycast_kernel<lw::FieldWarp>"}[dom]
     roofline = {"bound": "valu", "kernel": f"void {kname}(RaycastParams)",
                 "note": "compute-bound on FP32 vector ALUs (no matrix cores); peak = MI355X FP32 157.3 TFLOP/s",

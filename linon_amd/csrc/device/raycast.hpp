@@ -343,8 +343,10 @@ struct Rgb {
 // Steps of one sample ray from p along d: the position before every stride-th step recorded, nsamp
 // of them.  One wave runs this for thousands of dependent steps, so its length in instructions is
 // a small frame's time: the records are counted down rather than found by dividing the step index
-// (about 30 instructions a step; swirl's 5000 steps 1.26 -> 0.95 ms, hot air's 4.0 -> 3.5), and
-// nothing is integrated past the last one.  One loop for every field weight: a second one for
+// (about 30 instructions a step; swirl's 5000 steps 1.22 -> 0.98 ms), and nothing is integrated past
+// the last one.  Alone on its SIMD the wave issues a vector instruction every 6 to 7 cycles (swirl 85 a
+// step, hot air's default variant 289, the spherical sigmoid mirage 462): the latency of one upon
+// another, not the rate of issue.  One loop for every field weight: a second one for
 // weight 1 saves six instructions a step here but slows the pixels' loop of the same kernel by
 // 2.5% (1080p hot air 13.6 -> 13.95 ms).
 template <class F>

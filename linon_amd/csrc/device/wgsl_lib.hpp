@@ -416,9 +416,11 @@ __device__ __forceinline__ vec3 refraction_impl(float t_in, float t_out, vec3 v_
     // v_i, RN(X n_ref_i)), X = fma(eta, |cosi|, -sqrt(k)) (the form the compiler picked for the
     // expression); with n, X n_ref = Y n, Y = fma(-eta, cosi, +-sqrt(k)), the root negated where cosi
     // < 0.  One select instead of a branch over the side: its exec mask and moves took about 25 cycles
-    // a stage where a wave has its SIMD to itself (a 96x64 frame of the spherical sigmoid mirage, all
-    // sample rays, 5.3 -> 4.9 ms; 1080p hot air 13.55 -> 13.47 ms, plane mirage 13.55 -> 12.48).  With
-    // copysign(root, cosi) in place of the select, 1080p hot air takes 13.85.  NaN where k < 0.
+    // a stage where a wave has its SIMD to itself; 1080p plane mirage 13.55 -> 12.48 ms.  (The 5000 steps
+    // of the sample rays, their shorter bookkeeping included: the spherical mirage 5.74 -> 4.99 ms, with
+    // sigmoid 6.85 -> 6.44, hot air's default variant 3.98 -> 3.65.)  Where a loop is faster with the
+    // branch, loop_fields.hpp says so.  With copysign(root, cosi) in place of the select, 1080p hot air
+    // takes 13.85 ms where it takes 13.47.  NaN where k < 0.
     const float root = sqrt_rn_no_tiny(k);
     const float Y = SideBranch ? __builtin_fmaf(eta, cosi, -root)
                                : __builtin_fmaf(-eta, cosi, cosi < 0.0f ? -root : root);

@@ -44,6 +44,6 @@ enum class GridResult {
     FAILED      // any other error of HIP's
 };
 GridResult build_grid_device(const GridGeom& g, const float* h_xyz, uint32_t nv, const uint32_t* h_faces, uint32_t nf,
-                       hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err);
+                             hipStream_t s, int refuse_alloc, DeviceGrid& out, std::string& err);
 
 }  // namespace linon
