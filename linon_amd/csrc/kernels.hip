@@ -338,6 +338,11 @@ __global__ void __launch_bounds__(256) div_selftest_refraction_kernel(unsigned l
     // one temperature on both sides: refraction_in_range_same against the general form
     const lw::vec3 c = lw::refraction_in_range_same(t_in, v, nrm), d = lw::refraction_in_range(t_in, t_in, v, nrm);
     bad += !same_or_nan(c.x, d.x) + !same_or_nan(c.y, d.y) + !same_or_nan(c.z, d.z);
+    // both by the branch over the side of the surface, which some step loops run
+    const lw::vec3 ab = lw::refraction_in_range<true>(t_in, t_out, v, nrm);
+    const lw::vec3 cb = lw::refraction_in_range_same<true>(t_in, v, nrm);
+    bad += !same_or_nan(ab.x, b.x) + !same_or_nan(ab.y, b.y) + !same_or_nan(ab.z, b.z);
+    bad += !same_or_nan(cb.x, c.x) + !same_or_nan(cb.y, c.y) + !same_or_nan(cb.z, c.z);
     // the refracting fields' first RK4 stage, f.first_stage(p, v0, v, t) = f(p, p, v0, v, t),
     // with p taken from the random normals (components in [-1.5, 1.5])
     bad += first_stage_mismatches(lw::FieldHotAir{}, nrm, v);
@@ -513,7 +518,7 @@ hipError_t run_division_selftest(unsigned long long random_pairs, unsigned long 
             const unsigned long long m = random_pairs - off < chunk ? random_pairs - off : chunk;
             hipLaunchKernelGGL(div_selftest_refraction_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0,
                                nullptr, 0x5851F42D4C957F2Dull + off, m, d + 1);
-            n += 29 * m;
+            n += 35 * m;
         }
         for (unsigned long long off = 0; off < random_pairs && e == hipSuccess; off += chunk) {
             const unsigned long long m = random_pairs - off < chunk ? random_pairs - off : chunk;
