@@ -11,7 +11,7 @@
 // It is deliberately naive: brute force over all faces in index order, exactly as
 // `ray_color` (src/main_view.wgsl:177-220) does it.  Nothing in the product library
 // links or calls this file; only tests/, the smoke check and bench.py's CPU-baseline leg
-// load it (through ctypes) as the checker.
+// load it (through ctypes), for results to compare with.
 //
 // Parity pins for each function live in tests/test_oracle_*.py; the functions without a
 // pin independent of this file are listed in the module docstring of oracle/oracle.py.

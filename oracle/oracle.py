@@ -1,7 +1,7 @@
 """ctypes wrapper of the CPU oracle (liblinon_oracle.so) — TEST INFRASTRUCTURE ONLY.
 
 Only tests/, the smoke check of __graft_entry__.py and the CPU-baseline leg of bench.py use
-this module, always as the checker; the product library never loads it.
+this module, always for results to compare with; the product library never loads it.
 
 What pins each oracle function (tests/test_oracle_pins.py unless noted):
   hit_triangle       textbook known answers (centroid, edges/vertices inclusive, parallel,
